@@ -1217,7 +1217,14 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             q.x = s->X; q.x_stride = c.dim; q.cols = c.dim; q.n = mt;
             q.norm_w = y.attn_norm; q.eps = c.norm_eps;
             if (l == 0) { q.ids = s->ids_d; q.emb = m->emb; q.x_out = s->X; }
-            q.xf = m->any_f32 ? s->xf : nullptr; q.qx = s->qx; q.dx = s->dxp; q.xs = s->xsum;
+            // the rows a product reads: fp32 for F32 weights, Q8_0 codes otherwise
+            const bool any_f32 = m->any_f32;
+            auto rows_for = [&](QuantRowsArgs &r, const DMat &W) {
+                const bool f = W.dtype == DT_F32;
+                r.xf = f ? s->xf : nullptr;
+                r.qx = f ? nullptr : s->qx; r.dx = s->dxp; r.xs = s->xsum;
+            };
+            rows_for(q, y.qkv);
             // copies of the captured layer's tensors of this pass
             const bool snap = l == s->pdbg_layer && pass == s->pdbg_pass;
             auto psnap = [&](int slot, const float *src, int stride, int width) -> int {
@@ -1248,7 +1255,7 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             // k_pf_kvsplit)
             const bool img_ok = !exact && (hd == 64 || hd == 128) && s->pf_kvimg && pos0 % 64 == 0 &&
                                 s->pf_kvimg_tiles >= (pos0 + mt + 63) / 64 && env_int("EHIP_PF_KVIMG", 1);
-            if (!q.xf && gemm_qkv_fits(g, p)) {
+            if (!any_f32 && gemm_qkv_fits(g, p)) {
                 // short prompts: the QK-norm, RoPE and cache stores in the
                 // product's epilogue (the raw product goes straight to a capture)
                 if (img_ok) {
@@ -1257,7 +1264,7 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
                     img_fused = true;
                 }
                 rc |= launch_gemm_qkv(s->st, s->f16kv, g, p, snap ? s->pdbg[DBG_QKV] : nullptr);
-            } else if (!q.xf && env_int("EHIP_PF_QKPOST", 1) && gemm_qkpost_fits(g, p)) {
+            } else if (!any_f32 && env_int("EHIP_PF_QKPOST", 1) && gemm_qkpost_fits(g, p)) {
                 // longer ones, 128-dim heads: the same in the matrix-core
                 // product's epilogue (EHIP_PF_QKPOST=0 keeps the product and
                 // k_qkpost apart)
@@ -1283,37 +1290,43 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             // the attention can quantize its own output for wo (not for F32
             // weights, whose product reads the fp32 rows)
             bool quantized = false;
-            if (!q.xf) { at.qx = s->qx; at.qdx = s->dxp; at.qxs = s->xsum; }
+            if (!any_f32) { at.qx = s->qx; at.qdx = s->dxp; at.qxs = s->xsum; }
             rc |= exact ? launch_attention(s->st, s->f16kv, at, &quantized)
                         : launch_attention_mfma(s->st, s->f16kv, at, &quantized);
             if (psnap(DBG_O, s->O, qd, qd)) return -1;
-            if (!quantized) {
-                QuantRowsArgs q2{};
-                q2.x = s->O; q2.x_stride = qd; q2.cols = qd; q2.n = mt;
-                q2.xf = q.xf; q2.qx = s->qx; q2.dx = s->dxp; q2.xs = s->xsum;
-                rc |= launch_quant_rows(s->st, q2);
-            }
             GemmArgs g2{};
             g2.W = y.wo; g2.units = c.dim; g2.n = mt; g2.qx = s->qx; g2.dx = s->dxp; g2.xs = s->xsum;
-            g2.xf = q.xf; g2.out = s->X; g2.out_stride = c.dim;
+            g2.xf = s->O; g2.out = s->X; g2.out_stride = c.dim;
+            if (!quantized && y.wo.dtype != DT_F32) {
+                QuantRowsArgs q2{};
+                q2.x = s->O; q2.x_stride = qd; q2.cols = qd; q2.n = mt;
+                rows_for(q2, y.wo);
+                rc |= launch_quant_rows(s->st, q2);
+            }
             rc |= launch_gemm(s->st, EPI_RESID, g2);
             if (psnap(DBG_XMID, s->X, c.dim, c.dim)) return -1;
             QuantRowsArgs q3 = q;
             q3.ids = nullptr; q3.norm_w = y.ffn_norm;
+            rows_for(q3, y.w13);
             rc |= launch_quant_rows(s->st, q3);
             GemmArgs g3{};
             g3.W = y.w13; g3.units = 2 * hid; g3.n = mt; g3.qx = s->qx; g3.dx = s->dxp; g3.xs = s->xsum;
-            g3.xf = q.xf; g3.out = s->H; g3.out_stride = 2 * hid;
+            g3.xf = q3.xf; g3.out = s->H; g3.out_stride = 2 * hid;
             GemmArgs g4{};
             g4.W = y.w2; g4.units = c.dim; g4.n = mt; g4.qx = s->qx; g4.dx = s->dxp; g4.xs = s->xsum;
             // the SwiGLU and its quantization in the w1|w3 product's epilogue
             // (the gate | up rows written only for a capture): the short-prompt
             // kernel, or the matrix-core tiles (EHIP_PF_SWIGLU=0 keeps those
-            // passes on the product + k_quant_rows)
+            // passes on the product + k_quant_rows); F32 weights on both
+            // sides: the SwiGLU rows, as the w2 product reads them
             GemmArgs gs = g3;
             gs.units = hid; gs.pair_off = hid; gs.oq = s->qx2; gs.odx = s->dxp2; gs.oxs = s->xsum2;
             gs.out = snap ? s->H : nullptr;
-            if (!q.xf && (gemm_swiglu_fits(gs) || (env_int("EHIP_PF_SWIGLU", 1) && gemm_swiglu_long_fits(gs)))) {
+            if (y.w13.dtype == DT_F32 && y.w2.dtype == DT_F32 && !snap) {
+                gs.out = s->H; gs.out_stride = hid;
+                rc |= launch_gemm(s->st, EPI_SWIGLU, gs);
+                g4.xf = s->H;
+            } else if (!any_f32 && (gemm_swiglu_fits(gs) || (env_int("EHIP_PF_SWIGLU", 1) && gemm_swiglu_long_fits(gs)))) {
                 rc |= launch_gemm_swiglu(s->st, gs);
                 if (psnap(DBG_H, s->H, 2 * hid, 2 * hid)) return -1;
                 g4.qx = s->qx2; g4.dx = s->dxp2; g4.xs = s->xsum2;
@@ -1322,10 +1335,11 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
                 if (psnap(DBG_H, s->H, 2 * hid, 2 * hid)) return -1;
                 QuantRowsArgs q4{};
                 q4.x = s->H; q4.x_stride = 2 * hid; q4.cols = hid; q4.n = mt; q4.swiglu = 1;
-                q4.xf = q.xf; q4.qx = s->qx; q4.dx = s->dxp; q4.xs = s->xsum;
+                rows_for(q4, y.w2);
                 rc |= launch_quant_rows(s->st, q4);
+                g4.xf = q4.xf;
             }
-            g4.xf = q.xf; g4.out = s->X; g4.out_stride = c.dim;
+            g4.out = s->X; g4.out_stride = c.dim;
             rc |= launch_gemm(s->st, EPI_RESID, g4);
             if (psnap(DBG_XOUT, s->X, c.dim, c.dim)) return -1;
             if (rc) { set_err("a prefill kernel could not be launched for this shape"); return -1; }

@@ -1,0 +1,69 @@
+"""F32 weights: the products on the fp32 matrix cores against float64 on the
+GPU's own inputs, at the edges of their tiles.
+
+Bound per output: kernel_check's for float32 sums, 1e-6 of sum |w||x| plus
+two ulps of the result.  Of an output's K terms a wave adds K / 4 in a chain,
+so K / 4 roundings of at most 2^-24 of the partial sum, which walk like their
+square root: at K = 2080 about 23 x 6e-8 = 1.4e-6 of a partial sum that is
+itself near sum |w||x| / K^0.5, far below the bound.
+"""
+import numpy as np
+import pytest
+
+import kernel_check as kc
+from emberllm_amd import _native, configs, emberllm
+
+pytestmark = pytest.mark.gpu
+
+
+def model(name, dim, hidden, heads, kv, hd, bias):
+    cfg = dict(configs.TINY["t_f32"], dim=dim, hidden_dim=hidden, n_heads=heads, n_kv_heads=kv, head_dim=hd,
+               qkv_bias=bias, max_seq_len=1024)
+    return configs.model_path("f32w_" + name, cfg)
+
+
+def check(rep, name, W, x, out, pre=None, bias=None):
+    y, mag = np.empty((len(x), W.rows)), np.empty((len(x), W.rows))
+    x = x.astype(np.float64)
+    r0 = 0
+    for r0, w in W.chunks():
+        y[:, r0:r0 + len(w)] = x @ w.T
+        mag[:, r0:r0 + len(w)] = np.abs(x) @ np.abs(w).T
+    if bias is not None:
+        y += bias
+    if pre is not None:
+        y += pre
+    rep.add(name, out, y, kc.SUM_TOL * mag + 2 * kc.F32_ULP * np.abs(y) + 1e-30)
+
+
+# K of 3 blocks (a wave without any), 25 (uneven quarters) and 65; outputs and
+# tokens that end inside a tile; the last two reach the 64 x 64 tiles
+SHAPES = [("t", 96, 192, 2, 1, 48, 0), ("u", 800, 1056, 16, 8, 64, 1), ("v", 2080, 608, 2, 1, 64, 0)]
+
+
+@pytest.mark.parametrize("shape,n", [(s, n) for s in SHAPES for n in (2, 31, 33, 70)] + [(SHAPES[1], 1000), (SHAPES[2], 1000)],
+                         ids=lambda v: v[0] if isinstance(v, tuple) else str(v))
+def test_prefill_products(shape, n):
+    path = model(*shape)
+    mf = kc.ModelFile(path)
+    eng = emberllm.Engine(path, ctx=1024)
+    ids = np.random.default_rng(n).integers(0, mf.V, n)
+    got = []
+    for layer in (0, 1):
+        eng.debug_capture_prefill(layer, 0)
+        eng.prefill(ids)
+        got.append([np.asarray(eng.debug_read_prefill(s)[0]) for s in range(6)])
+    eng.debug_capture_prefill(-1, 0)
+    eng.close()
+    xin, qkv, o, xmid, h13, xout = got[0]
+    rep = kc.Report(f"{shape[0]} n {n}")
+    bias = np.concatenate([mf.vec(f"layers.0.{w}_bias") for w in ("wq", "wk", "wv")]) if shape[6] else None
+    check(rep, "qkv", mf.mat(mf.layer(0, "qkv")), kc.rmsnorm_f32(xin, mf.vec("layers.0.attn_norm"), mf.eps), qkv, bias=bias)
+    check(rep, "wo", mf.mat(mf.layer(0, "wo")), o, xmid, pre=xin)
+    check(rep, "w1|w3", mf.mat(mf.layer(0, "w13")), kc.rmsnorm_f32(xmid, mf.vec("layers.0.ffn_norm"), mf.eps), h13)
+    check(rep, "w2", mf.mat(mf.layer(0, "w2")), kc.swiglu_f32(h13, mf.hid), xout, pre=xmid)
+    print(rep, flush=True)
+    assert rep.ok, str(rep)
+    # the second run's layer 0 had its SwiGLU in the w1|w3 product, the first
+    # run's as a kernel of its own: the same sums, the same function
+    np.testing.assert_array_equal(got[1][0], xout)
