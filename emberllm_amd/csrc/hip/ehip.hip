@@ -892,16 +892,16 @@ __global__ void k_step_done(const int *tokpos, int *done_h) {
 }
 
 // One API decode step: token, position and ticket in (one 16-byte copy), the
-// layers, the head, the logits out, the ticket back.  The quantized heads
-// store the logits (and the error flag behind them) straight into the pinned
-// host buffer as they are produced, so the PCIe writes overlap the head's
-// weight stream (a copy after the head added about 12 us per step); the F32
-// and reference-order heads are followed by a copy.
+// layers, the head, the logits out, the ticket back.  The head stores the
+// logits (and the error flag behind them) straight into the pinned host
+// buffer as they are produced, so the PCIe writes overlap its weight stream
+// (a copy after the head added about 12 us per step); the reference-order
+// head is followed by a copy.
 static int enq_step(EhipState *s) {
     const int V = s->m->cfg.vocab_size;
     HCHK(hipMemcpyAsync(s->tokpos_d, s->tokpos_h, 16, hipMemcpyHostToDevice, s->st), -1);
     if (enq_layers(s)) { set_err("a decode kernel could not be launched for this shape"); return -1; }
-    const bool direct = !s->ref_order && s->m->head.dtype != DT_F32;
+    const bool direct = !s->ref_order;
     MatvecArgs a = head_args(s, x_final(s));
     if (direct) a.out_host = s->logits_h;
     if (mv(s, PRO_NORM, EPI_STORE, a)) { set_err("lm_head launch failed"); return -1; }

@@ -342,56 +342,161 @@ __global__ __launch_bounds__(WG) void k_matvec(MatvecArgs a) {
     }
 }
 
-// F32 weights (files the reference leaves unquantized, quant.c:26-57): plain
-// fp32 dot products in the reference's order (dot_f32, kernels.c:120-135),
-// the activation kept in LDS.
-template <int PRO, int EPI>
+// F32 weights (files the reference leaves unquantized, quant.c:26-57;
+// dot_f32, kernels.c:120-135), with k_matvec's schedule: the activation's
+// loads, then the first row group's weights, issued before either is used,
+// and further groups prefetched.  A wave walks its UPW outputs' rows in
+// segments of NCH 16-byte chunks per lane (lane l chunks l, l + 64, ...), one
+// segment per row for K <= 256 NCH; the activation stays in LDS, since a
+// segment of it serves UPW rows.  XPT: float4 slots of the activation per
+// thread, loaded together; 0 for K > 2048, whose prologue loops.
+// Bound: a launch's memory round trips, then the weights' stream (2.4-12.6 MB
+// per product of the stories110M shape): q|k|v 6.9 -> 3.7 us, w1|w3 8.1 ->
+// 4.8, wo 3.1 and w2 4.1 (6.9 on average before), head (98 MB) 20.1 -> 17.4
+// against a loop of load-use pairs behind the activation's prologue; the
+// step at position 300, its logits stored to the host by the head, 450 -> 301.
+template <int PRO, int EPI, int NCH, int UPW, int XPT>
 __global__ __launch_bounds__(WG) void k_matvec_f32(MatvecArgs a) {
+    constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1, XN = XPT ? XPT : 1;
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ float red[NWAVE];
-    const int K = a.W.cols;
-    float *xs = reinterpret_cast<float *>(smem);
+    const int K = a.W.cols, nch = K / 4, nseg = (nch + 64 * NCH - 1) / (64 * NCH);
+    f32x4 *xs = reinterpret_cast<f32x4 *>(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float ss = 0.0f;
-    for (int i = tid; i < K; i += WG) {
-        float v;
-        if (PRO == PRO_EMBED_NORM) {
-            const int tok = a.tokpos[0];
-            v = a.emb.dtype == DT_F32 ? reinterpret_cast<const float *>(a.emb.q)[(size_t)tok * K + i]
-                                      : (float)reinterpret_cast<const int8_t *>(a.emb.q)[(size_t)tok * K + i] *
-                                            h2f(a.emb.d[(size_t)tok * (K / QB) + i / QB]);
-            if (blockIdx.x == 0) a.x_out[i] = v;
-        } else {
-            v = a.in[i];
+    const int nw = gridDim.x * NWAVE;
+    int u0 = (blockIdx.x * NWAVE + wave) * UPW;
+
+    // ---- activation (issued first), then the first segment's weights
+    const bool emb_q = PRO == PRO_EMBED_NORM && a.emb.dtype != DT_F32;
+    const int tok = PRO == PRO_EMBED_NORM ? a.tokpos[0] : 0;
+    const f32x4 *in4 = PRO == PRO_EMBED_NORM ? reinterpret_cast<const f32x4 *>(a.emb.q) + (size_t)tok * nch
+                                             : reinterpret_cast<const f32x4 *>(a.in);
+    auto fetch = [&](int s) __attribute__((always_inline)) -> f32x4 {
+        if (!emb_q) return in4[s];
+        const int q = reinterpret_cast<const int *>(a.emb.q + (size_t)tok * K)[s];
+        const float d = h2f(a.emb.d[(size_t)tok * (K / QB) + (s >> 3)]);
+        return f32x4{(float)(int8_t)(q & 0xff) * d, (float)(int8_t)((q >> 8) & 0xff) * d,
+                     (float)(int8_t)((q >> 16) & 0xff) * d, (float)(int8_t)(q >> 24) * d};
+    };
+    f32x4 xv[XN], nv[XN];
+    if constexpr (XPT > 0) {
+#pragma unroll
+        for (int i = 0; i < XPT; i++) xv[i] = fetch(min(tid + WG * i, nch - 1));
+        if constexpr (PRO != PRO_PLAIN) {
+#pragma unroll
+            for (int i = 0; i < XPT; i++) nv[i] = reinterpret_cast<const f32x4 *>(a.norm_w)[min(tid + WG * i, nch - 1)];
         }
-        xs[i] = v;
-        ss += v * v;
     }
-    if (PRO != PRO_PLAIN) {
-        const float tot = block_sum(ss, red);
-        const float scale = 1.0f / sqrtf(tot / (float)K + a.eps);
-        for (int i = tid; i < K; i += WG) xs[i] = xs[i] * scale * a.norm_w[i];
+    f32x4 cur[UPW][NR][NCH], nxt[UPW][NR][NCH];
+    float pre[UPW], prn[UPW];
+    auto load = [&](f32x4 (&w)[UPW][NR][NCH], float (&pr)[UPW], int u, int seg) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < UPW; j++) {
+            const int uc = min(u + j, a.units - 1);
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                const f32x4 *row = reinterpret_cast<const f32x4 *>(a.W.q) + (size_t)(uc + r * a.pair_off) * nch;
+#pragma unroll
+                for (int i = 0; i < NCH; i++) w[j][r][i] = row[min(lane + 64 * (seg * NCH + i), nch - 1)];
+            }
+            if (EPI == EPI_STORE) pr[j] = a.bias ? a.bias[uc] : 0.0f;
+            else if (EPI == EPI_RESID) pr[j] = a.out[uc];
+            else pr[j] = 0.0f;
+        }
+    };
+    load(cur, pre, u0, 0);
+
+    // ---- RMSNorm, the activation into LDS
+    auto sq = [](f32x4 v) { return v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; };
+    float ss = 0.0f;
+    if constexpr (XPT > 0) {
+#pragma unroll
+        for (int i = 0; i < XPT; i++)
+            if (tid + WG * i < nch) ss += sq(xv[i]);
+    } else {
+        for (int s = tid; s < nch; s += WG) { const f32x4 v = fetch(s); xs[s] = v; ss += sq(v); }
+    }
+    if (PRO == PRO_EMBED_NORM && blockIdx.x == 0)
+        for (int s = tid; s < nch; s += WG) reinterpret_cast<f32x4 *>(a.x_out)[s] = fetch(s);
+    float scale = 1.0f;
+    if (PRO != PRO_PLAIN) scale = 1.0f / sqrtf(block_sum(ss, red) / (float)K + a.eps);   // model.c:50-55
+    if constexpr (XPT > 0) {
+#pragma unroll
+        for (int i = 0; i < XPT; i++) {
+            if constexpr (PRO != PRO_PLAIN) xv[i] = xv[i] * scale * nv[i];
+            if (tid + WG * i < nch) xs[tid + WG * i] = xv[i];
+        }
+    } else if (PRO != PRO_PLAIN) {
+        for (int s = tid; s < nch; s += WG) xs[s] = xs[s] * scale * reinterpret_cast<const f32x4 *>(a.norm_w)[s];
     }
     __syncthreads();
-    constexpr int NR = EPI == EPI_SWIGLU ? 2 : 1;
-    const int gw = blockIdx.x * NWAVE + wave, nw = gridDim.x * NWAVE;
-    const float4 *x4 = reinterpret_cast<const float4 *>(xs);
-    for (int u = gw; u < a.units; u += nw) {
-        float v[NR];
+
+    // the error-flag word behind the outputs, for the host's copy
+    if (EPI == EPI_STORE && a.out_host && blockIdx.x == 0 && tid == 0)
+        reinterpret_cast<int *>(a.out_host)[a.units] = reinterpret_cast<const int *>(a.out)[a.units];
+
+    // ---- row groups, segment by segment, the next one's loads in flight
+    f32x4 acc[UPW][NR];
+    for (int seg = 0; u0 < a.units;) {
+        const bool end = seg + 1 == nseg;
+        const int un = end ? u0 + nw * UPW : u0, sn = end ? 0 : seg + 1;
+        if (un < a.units) load(nxt, prn, un, sn);
 #pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const float4 *wrow = reinterpret_cast<const float4 *>(a.W.q) + (size_t)(u + r * a.pair_off) * (K / 4);
-            float s = 0.0f;
-            for (int c = lane; c < K / 4; c += 64) {
-                const float4 w = wrow[c], x = x4[c];
-                s += w.x * x.x + w.y * x.y + w.z * x.z + w.w * x.w;
-            }
-            v[r] = wave_sum(s);
+        for (int i = 0; i < NCH; i++) {
+            const int c = lane + 64 * (seg * NCH + i);
+            const f32x4 x = xs[min(c, nch - 1)];
+#pragma unroll
+            for (int j = 0; j < UPW; j++)
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    const f32x4 was = seg + i ? acc[j][r] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    f32x4 t;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) t[e] = fmaf(cur[j][r][i][e], x[e], was[e]);
+                    acc[j][r] = c < nch ? t : was;
+                }
         }
-        if (lane == 0) {
-            if (EPI == EPI_STORE) a.out[u] = a.bias ? v[0] + a.bias[u] : v[0];
-            else if (EPI == EPI_RESID) a.out[u] += v[0];
-            else { const float g = v[0]; a.out[u] = g / (1.0f + expf(-g)) * v[NR - 1]; }
+        if (end) {
+            float v[UPW][NR], mine[NR], p = pre[0];
+#pragma unroll
+            for (int j = 0; j < UPW; j++)
+#pragma unroll
+                for (int r = 0; r < NR; r++)
+                    v[j][r] = wave_sum((acc[j][r].x + acc[j][r].y) + (acc[j][r].z + acc[j][r].w));
+#pragma unroll
+            for (int r = 0; r < NR; r++) mine[r] = v[0][r];
+#pragma unroll
+            for (int j = 1; j < UPW; j++)
+                if (lane == j) {
+#pragma unroll
+                    for (int r = 0; r < NR; r++) mine[r] = v[j][r];
+                    p = pre[j];
+                }
+            const int u = u0 + lane;
+            if (lane < UPW && u < a.units) {
+                if (EPI == EPI_STORE) {
+                    const float o = a.bias ? mine[0] + p : mine[0];
+                    a.out[u] = o;
+                    if (a.out_host) a.out_host[u] = o;
+                } else if (EPI == EPI_RESID) {
+                    a.out[u] = p + mine[0];
+                } else {
+                    const float g = mine[0];
+                    a.out[u] = g / (1.0f + expf(-g)) * mine[NR - 1];
+                }
+            }
+        }
+        u0 = un;
+        seg = sn;
+        if (un < a.units) {
+#pragma unroll
+            for (int j = 0; j < UPW; j++) {
+                pre[j] = prn[j];
+#pragma unroll
+                for (int r = 0; r < NR; r++)
+#pragma unroll
+                    for (int i = 0; i < NCH; i++) cur[j][r][i] = nxt[j][r][i];
+            }
         }
     }
 }
@@ -441,6 +546,37 @@ static int pick_nch(hipStream_t st, const MatvecArgs &a, size_t lds) {
     return -1;
 }
 
+// F32: the largest of 4, 2, 1 outputs per wave that still gives every CU a
+// workgroup, as above (two rows each for the SwiGLU: at most 2); chunks per
+// segment by K (a longer row in segments of 8)
+template <int PRO, int EPI, int NCH, int XPT>
+static int go_f32(hipStream_t st, const MatvecArgs &a) {
+#define GOF(UPW)                                                                                                \
+    {                                                                                                           \
+        const int grid = grid_for(a.units, UPW);                                                                \
+        hipLaunchKernelGGL((k_matvec_f32<PRO, EPI, NCH, UPW, XPT>), dim3(grid), dim3(WG), (size_t)a.W.cols * 4, st, a); \
+        return grid;                                                                                            \
+    }
+    if constexpr (NCH <= 4 && EPI != EPI_SWIGLU) {
+        if (a.units >= 4 * NWAVE * 256) GOF(4)
+    }
+    if constexpr (NCH <= 4) {
+        if (a.units >= 2 * NWAVE * 256) GOF(2)
+    }
+    GOF(1)
+#undef GOF
+}
+
+template <int PRO, int EPI>
+static int pick_f32(hipStream_t st, const MatvecArgs &a) {
+    const int K = a.W.cols;
+    if (K <= 512) return go_f32<PRO, EPI, 2, 1>(st, a);
+    if (K <= 768) return go_f32<PRO, EPI, 3, 1>(st, a);
+    if (K <= 1024) return go_f32<PRO, EPI, 4, 1>(st, a);
+    if (K <= 2048) return go_f32<PRO, EPI, 8, 2>(st, a);
+    return go_f32<PRO, EPI, 8, 0>(st, a);
+}
+
 template <int PRO, int EPI>
 static int pick_dt(hipStream_t st, const MatvecArgs &a) {
     const int K = a.W.cols;
@@ -448,12 +584,10 @@ static int pick_dt(hipStream_t st, const MatvecArgs &a) {
         case DT_Q8: return pick_nch<DT_Q8, PRO, EPI>(st, a, (size_t)K + (size_t)(K / QB) * 8);
         case DT_Q4: return pick_nch<DT_Q4, PRO, EPI>(st, a, (size_t)K + (size_t)(K / QB) * 8);
         case DT_F32: {
-            if constexpr (PRO == PRO_NORM_PARTS) return -1;
-            if ((size_t)K * 4 > 64 * 1024) return -1;
-            long grid = ((long)a.units + NWAVE - 1) / NWAVE;
-            if (grid > MATVEC_MAX_GRID) grid = MATVEC_MAX_GRID;
-            hipLaunchKernelGGL((k_matvec_f32<PRO, EPI>), dim3(grid), dim3(WG), (size_t)K * 4, st, a);
-            return (int)grid;
+            if constexpr (PRO != PRO_NORM_PARTS) {
+                if ((size_t)K * 4 <= 64 * 1024) return pick_f32<PRO, EPI>(st, a);
+            }
+            return -1;
         }
     }
     return -1;
@@ -463,7 +597,7 @@ int launch_matvec(hipStream_t st, int pro, int epi, const MatvecArgs &a) {
     const int K = a.W.cols;
     if (K % QB != 0 || K <= 0 || a.units <= 0) return -1;
     if (a.am_val && (epi != EPI_STORE || a.W.dtype == DT_F32)) return -1;
-    if (a.out_host && (epi != EPI_STORE || a.W.dtype == DT_F32)) return -1;
+    if (a.out_host && epi != EPI_STORE) return -1;
     int grid = -1;
     if (pro == PRO_NORM && epi == EPI_STORE) grid = pick_dt<PRO_NORM, EPI_STORE>(st, a);
     else if (pro == PRO_EMBED_NORM && epi == EPI_STORE) grid = pick_dt<PRO_EMBED_NORM, EPI_STORE>(st, a);

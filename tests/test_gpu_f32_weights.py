@@ -1,5 +1,6 @@
-"""F32 weights: the products on the fp32 matrix cores against float64 on the
-GPU's own inputs, at the edges of their tiles.
+"""F32 weights: the prompt's products on the fp32 matrix cores and the decode
+step's matvecs against float64 on the GPU's own inputs, at the edges of their
+tiles and row segments.
 
 Bound per output: kernel_check's for float32 sums, 1e-6 of sum |w||x| plus
 two ulps of the result.  Of an output's K terms a wave adds K / 4 in a chain,
@@ -16,9 +17,9 @@ from emberllm_amd import _native, configs, emberllm
 pytestmark = pytest.mark.gpu
 
 
-def model(name, dim, hidden, heads, kv, hd, bias):
+def model(name, dim, hidden, heads, kv, hd, bias, vocab=320):
     cfg = dict(configs.TINY["t_f32"], dim=dim, hidden_dim=hidden, n_heads=heads, n_kv_heads=kv, head_dim=hd,
-               qkv_bias=bias, max_seq_len=1024)
+               qkv_bias=bias, max_seq_len=1024, vocab_size=vocab)
     return configs.model_path("f32w_" + name, cfg)
 
 
@@ -67,3 +68,39 @@ def test_prefill_products(shape, n):
     # the second run's layer 0 had its SwiGLU in the w1|w3 product, the first
     # run's as a kernel of its own: the same sums, the same function
     np.testing.assert_array_equal(got[1][0], xout)
+
+
+# a row of 24 chunks (part of a wave), of 200, of 520 (two segments of 8 x 64
+# chunks, the second short, with the looped activation prologue) and the
+# widths of each segment size; the vocabulary's rows four to a wave
+DECODE = SHAPES + [("w", 512, 768, 8, 4, 64, 0), ("x", 1024, 2048, 2, 1, 64, 1)]
+
+
+@pytest.mark.parametrize("shape", DECODE, ids=lambda v: v[0])
+def test_decode_products(shape):
+    path = model(*shape, vocab=4101)
+    mf = kc.ModelFile(path)
+    eng = emberllm.Engine(path, ctx=1024)
+    eng.prefill(np.arange(5))
+    rep = kc.Report(shape[0])
+    for step, layer in enumerate((0, 1)):
+        eng.debug_capture(layer)
+        logits = eng.forward(40 + step, 5 + step)
+        xin, qkv, o, xmid, h, xout = (eng.debug_read(s)[None] for s in range(6))
+        p = f"layers.{layer}."
+        bias = np.concatenate([mf.vec(p + w + "_bias") for w in ("wq", "wk", "wv")]) if shape[6] else None
+        check(rep, f"L{layer} qkv", mf.mat(mf.layer(layer, "qkv")), kc.rmsnorm_f32(xin, mf.vec(p + "attn_norm"), mf.eps), qkv, bias=bias)
+        check(rep, f"L{layer} wo", mf.mat(mf.layer(layer, "wo")), o, xmid, pre=xin)
+        x = kc.rmsnorm_f32(xmid, mf.vec(p + "ffn_norm"), mf.eps).astype(np.float64)
+        w = np.concatenate([c for _, c in mf.mat(mf.layer(layer, "w13")).chunks()])
+        g, u = (x @ w.T)[:, :mf.hid], (x @ w.T)[:, mf.hid:]
+        mg, mu = (np.abs(x) @ np.abs(w).T)[:, :mf.hid], (np.abs(x) @ np.abs(w).T)[:, mf.hid:]
+        sg = 1.0 / (1.0 + np.exp(-g))
+        bound = kc.SUM_TOL * (np.abs(sg * (1.0 + g * (1.0 - sg)) * u) * mg + np.abs(g * sg) * mu) + 8 * kc.F32_ULP * np.abs(g * sg * u) + 1e-30
+        rep.add(f"L{layer} swiglu", h, g * sg * u, bound)
+        check(rep, f"L{layer} w2", mf.mat(mf.layer(layer, "w2")), h, xout, pre=xmid)
+    check(rep, "head", mf.mat(mf.head_names()), kc.rmsnorm_f32(xout, mf.vec("final_norm"), mf.eps), logits[None])
+    eng.debug_capture(-1)
+    eng.close()
+    print(rep, flush=True)
+    assert rep.ok, str(rep)
