@@ -1210,6 +1210,7 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
     const EhipConfig &c = m->cfg;
     const int hd = c.head_dim, qd = c.n_heads * hd, kvd = c.n_kv_heads * hd, hid = c.hidden_dim;
     const int stride = qd + 2 * kvd;
+    const bool few_ok = !s->pf_seq && env_int("EHIP_PF_FEW", 1);   // (0: the longer passes' kernels)
     {
         for (int l = 0; l < c.n_layers; l++) {
             const DevLayer &y = m->layers[l];
@@ -1235,7 +1236,9 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             };
             if (snap) { s->pdbg_n = mt; s->pdbg_pos = pos0; }
             if (l > 0 && psnap(DBG_XIN, s->X, c.dim, c.dim)) return -1;
-            int rc = launch_quant_rows(s->st, q);
+            const bool few = few_ok && gemm_few_fits(FewShape{y.qkv, y.wo, y.w13, y.w2, hd, mt});
+            if (few) { q.qx = nullptr; q.norm_w = nullptr; }   // the products take the rows themselves
+            int rc = few && l > 0 ? 0 : launch_quant_rows(s->st, q);
             if (l == 0 && psnap(DBG_XIN, s->X, c.dim, c.dim)) return -1;   // the embedded rows
             GemmArgs g{};
             g.W = y.qkv; g.units = stride; g.n = mt; g.qx = s->qx; g.dx = s->dxp; g.xs = s->xsum; g.xf = q.xf;
@@ -1255,7 +1258,14 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             // k_pf_kvsplit)
             const bool img_ok = !exact && (hd == 64 || hd == 128) && s->pf_kvimg && pos0 % 64 == 0 &&
                                 s->pf_kvimg_tiles >= (pos0 + mt + 63) / 64 && env_int("EHIP_PF_KVIMG", 1);
-            if (!any_f32 && gemm_qkv_fits(g, p)) {
+            if (few) {
+                if (img_ok) {
+                    p.kvimg = s->pf_kvimg;
+                    p.kvimg_tiles = s->pf_kvimg_tiles;
+                    img_fused = true;
+                }
+                rc |= launch_few_qkv(s->st, s->f16kv, g, NormIn{s->X, y.attn_norm, c.norm_eps}, p, snap ? s->pdbg[DBG_QKV] : nullptr);
+            } else if (!any_f32 && gemm_qkv_fits(g, p)) {
                 // short prompts: the QK-norm, RoPE and cache stores in the
                 // product's epilogue (the raw product goes straight to a capture)
                 if (img_ok) {
@@ -1303,12 +1313,12 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
                 rows_for(q2, y.wo);
                 rc |= launch_quant_rows(s->st, q2);
             }
-            rc |= launch_gemm(s->st, EPI_RESID, g2);
+            rc |= few ? launch_few_resid(s->st, g2) : launch_gemm(s->st, EPI_RESID, g2);
             if (psnap(DBG_XMID, s->X, c.dim, c.dim)) return -1;
             QuantRowsArgs q3 = q;
             q3.ids = nullptr; q3.norm_w = y.ffn_norm;
             rows_for(q3, y.w13);
-            rc |= launch_quant_rows(s->st, q3);
+            if (!few) rc |= launch_quant_rows(s->st, q3);
             GemmArgs g3{};
             g3.W = y.w13; g3.units = 2 * hid; g3.n = mt; g3.qx = s->qx; g3.dx = s->dxp; g3.xs = s->xsum;
             g3.xf = q3.xf; g3.out = s->H; g3.out_stride = 2 * hid;
@@ -1326,6 +1336,10 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
                 gs.out = s->H; gs.out_stride = hid;
                 rc |= launch_gemm(s->st, EPI_SWIGLU, gs);
                 g4.xf = s->H;
+            } else if (few) {
+                rc |= launch_few_swiglu(s->st, gs, NormIn{s->X, y.ffn_norm, c.norm_eps});
+                if (psnap(DBG_H, s->H, 2 * hid, 2 * hid)) return -1;
+                g4.qx = s->qx2; g4.dx = s->dxp2; g4.xs = s->xsum2;
             } else if (!any_f32 && (gemm_swiglu_fits(gs) || (env_int("EHIP_PF_SWIGLU", 1) && gemm_swiglu_long_fits(gs)))) {
                 rc |= launch_gemm_swiglu(s->st, gs);
                 if (psnap(DBG_H, s->H, 2 * hid, 2 * hid)) return -1;
@@ -1340,7 +1354,7 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
                 g4.xf = q4.xf;
             }
             g4.out = s->X; g4.out_stride = c.dim;
-            rc |= launch_gemm(s->st, EPI_RESID, g4);
+            rc |= few ? launch_few_resid(s->st, g4) : launch_gemm(s->st, EPI_RESID, g4);
             if (psnap(DBG_XOUT, s->X, c.dim, c.dim)) return -1;
             if (rc) { set_err("a prefill kernel could not be launched for this shape"); return -1; }
         }

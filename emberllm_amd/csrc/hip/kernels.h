@@ -283,6 +283,16 @@ bool gemm_qkpost_fits(const GemmArgs &g, const QkPostArgs &p);
 int launch_gemm_qkpost(hipStream_t st, bool f16kv, const GemmArgs &a, const QkPostArgs &p);
 int launch_gemm_qkv(hipStream_t st, bool f16kv, const GemmArgs &g, const QkPostArgs &p, float *raw);
 
+// The products of a pass of few tokens (gemm_few.hip), for layers whose four
+// matrices are all quantized and whose shapes gemm_few_fits: the q|k|v and
+// w1|w3 products normalize and quantize the rows x themselves.
+struct NormIn { const float *x; const float *norm_w; float eps; };   // x: [n][W.cols]
+struct FewShape { DMat qkv, wo, w13, w2; int hd, n; };
+bool gemm_few_fits(const FewShape &s);
+int launch_few_qkv(hipStream_t st, bool f16kv, const GemmArgs &a, const NormIn &in, const QkPostArgs &p, float *raw);
+int launch_few_swiglu(hipStream_t st, const GemmArgs &a, const NormIn &in);
+int launch_few_resid(hipStream_t st, const GemmArgs &a);   // EPI_RESID over rows quantized before
+
 // ---------------------------------------------------------------- sample --
 // Greedy selection (first maximum) over n logits; writes tokpos[0] = token,
 // tokpos[1] += 1 and appends the token to out[tokpos[2]++] (when < cap).
