@@ -29,6 +29,7 @@
 // -ffp-contract=off build.
 #include <cstdlib>
 
+#include <algorithm>
 #include "kernels.h"
 #include "flimg.h"
 
@@ -1007,108 +1008,118 @@ size_t attn_kvimg_bytes(int hd, bool f16kv, int ctx, int n_kv) {
     return 0;
 }
 
-// grid (kv heads, tiles of the pass's keys [0, pos_base + n_tok))
-template <int HD, bool F16>
-__global__ __launch_bounds__(WG) void k_pf_kvsplit(AttnArgs a) {
+// One (kv head, 64-key tile) of the cache by 256 threads: its rows from
+// position k0 into registers (load), then its image into LDS (image; K part
+// and exponents at kimg, V part at vimg).
+template <bool F16> struct FlQuad { typedef f32x4 type; };
+template <> struct FlQuad<true> { typedef uint2 type; };
+template <int HD, bool F16> struct FlTile {
     using I = FlImg<HD, F16>;
-    constexpr int NC = HD / 32;         // dim quads per lane and key
-    __shared__ __align__(16) uint8_t img[I::HBYTES];   // the image as it goes to HBM
-    uint8_t *vimg = img + I::KE;
-    int *kex = reinterpret_cast<int *>(img + I::KBYTES), *vex = kex + FL_BK;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = blockIdx.x, kt = blockIdx.y;
-    const int klast = a.pos_base + a.n_tok - 1;
-    const size_t hoff = (size_t)g * HD;
-    const int k0 = kt * FL_BK;
-    const int kp = 8 * wave + (lane & 7), dq0 = lane >> 3;
-    if constexpr (F16) {
-        uint2 kr[2][NC], vr[2][NC];
+    using quad = typename FlQuad<F16>::type;
+    static constexpr int NC = HD / 32;         // dim quads per lane and key
+    quad kr[2][NC], vr[2][NC];
+    __device__ __forceinline__ void load(const AttnArgs &a, int g, int k0, int klast, int tid) {
+        const size_t hoff = (size_t)g * HD;
+        const int kp = 8 * (tid >> 6) + (tid & 7), dq0 = (tid & 63) >> 3;
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int c = 0; c < NC; c++) {
                 const size_t off = (size_t)min(k0 + 2 * kp + j, klast) * a.kv_dim + hoff + 4 * (dq0 + 8 * c);
-                kr[j][c] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.kc) + off);
-                vr[j][c] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.vc) + off);
+                if constexpr (F16) {
+                    kr[j][c] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.kc) + off);
+                    vr[j][c] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(a.vc) + off);
+                } else {
+                    kr[j][c] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(a.kc) + off);
+                    vr[j][c] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(a.vc) + off);
+                }
             }
-        // dim quad dq = dq0 + 8c is half (dq & 1) of piece dq >> 1 of its K row;
-        // keys 2kp, 2kp + 1 are word kp & 3 of piece kp >> 2 of a V^T row
+    }
+    __device__ __forceinline__ void image(uint8_t *kimg, uint8_t *vimg, int tid) const {
+        const int kp = 8 * (tid >> 6) + (tid & 7), dq0 = (tid & 63) >> 3;
+        if constexpr (F16) {
+            // dim quad dq = dq0 + 8c is half (dq & 1) of piece dq >> 1 of its K row;
+            // keys 2kp, 2kp + 1 are word kp & 3 of piece kp >> 2 of a V^T row
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const int dq = dq0 + 8 * c;
+                    *reinterpret_cast<uint2 *>(kimg + I::k_at(fl_krow(2 * kp + j), dq >> 1) + 8 * (dq & 1)) = kr[j][c];
+                }
 #pragma unroll
             for (int c = 0; c < NC; c++) {
-                const int dq = dq0 + 8 * c;
-                *reinterpret_cast<uint2 *>(img + I::k_at(fl_krow(2 * kp + j), dq >> 1) + 8 * (dq & 1)) = kr[j][c];
+                const int d0 = 4 * (dq0 + 8 * c), w = 4 * (kp & 3);
+                const uint32_t r4[4] = { (vr[0][c].x & 0xffffu) | (vr[1][c].x << 16),
+                                         (vr[0][c].x >> 16) | (vr[1][c].x & 0xffff0000u),
+                                         (vr[0][c].y & 0xffffu) | (vr[1][c].y << 16),
+                                         (vr[0][c].y >> 16) | (vr[1][c].y & 0xffff0000u) };
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    *reinterpret_cast<uint32_t *>(vimg + I::v_at(d0 + e, kp >> 2) + w) = r4[e];
+            }
+        } else {
+            int *kex = reinterpret_cast<int *>(kimg + I::KBYTES), *vex = kex + FL_BK;
+            int ek[2], ev[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                float km = 0.0f, vm = 0.0f;
+#pragma unroll
+                for (int c = 0; c < NC; c++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        km = fmaxf(km, fabsf(kr[j][c][e]));
+                        vm = fmaxf(vm, fabsf(vr[j][c][e]));
+                    }
+                ek[j] = fl_exp(fl_pair_max(km));
+                ev[j] = fl_exp(fl_pair_max(vm));
+            }
+            if (dq0 == 0) {
+                kex[2 * kp] = ek[0]; kex[2 * kp + 1] = ek[1];
+                vex[2 * kp] = ev[0]; vex[2 * kp + 1] = ev[1];
             }
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const int d0 = 4 * (dq0 + 8 * c), w = 4 * (kp & 3);
-            const uint32_t r4[4] = { (vr[0][c].x & 0xffffu) | (vr[1][c].x << 16),
-                                     (vr[0][c].x >> 16) | (vr[1][c].x & 0xffff0000u),
-                                     (vr[0][c].y & 0xffffu) | (vr[1][c].y << 16),
-                                     (vr[0][c].y >> 16) | (vr[1][c].y & 0xffff0000u) };
+            for (int j = 0; j < 2; j++)
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                *reinterpret_cast<uint32_t *>(vimg + I::v_at(d0 + e, kp >> 2) + w) = r4[e];
-        }
-    } else {
-        f32x4 kr[2][NC], vr[2][NC];
+                for (int c = 0; c < NC; c++) {
+                    _Float16 hi[4], lo[4];
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const size_t off = (size_t)min(k0 + 2 * kp + j, klast) * a.kv_dim + hoff + 4 * (dq0 + 8 * c);
-                kr[j][c] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(a.kc) + off);
-                vr[j][c] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(a.vc) + off);
-            }
-        int ek[2], ev[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            float km = 0.0f, vm = 0.0f;
+                    for (int e = 0; e < 4; e++) {
+                        const float x = __builtin_amdgcn_ldexpf(kr[j][c][e], ek[j]);
+                        hi[e] = (_Float16)x;
+                        lo[e] = (_Float16)(x - (float)hi[e]);
+                    }
+                    const int dq = dq0 + 8 * c, rk = fl_krow(2 * kp + j);
+                    *reinterpret_cast<uint2 *>(kimg + I::k_at(rk, dq >> 1) + 8 * (dq & 1)) =
+                        make_uint2(fl_pack(hi[0], hi[1]), fl_pack(hi[2], hi[3]));
+                    *reinterpret_cast<uint2 *>(kimg + I::k_at(FL_BK + rk, dq >> 1) + 8 * (dq & 1)) =
+                        make_uint2(fl_pack(lo[0], lo[1]), fl_pack(lo[2], lo[3]));
+                }
 #pragma unroll
             for (int c = 0; c < NC; c++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    km = fmaxf(km, fabsf(kr[j][c][e]));
-                    vm = fmaxf(vm, fabsf(vr[j][c][e]));
+                    const float x0 = __builtin_amdgcn_ldexpf(vr[0][c][e], ev[0]);
+                    const float x1 = __builtin_amdgcn_ldexpf(vr[1][c][e], ev[1]);
+                    const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
+                    const _Float16 l0 = (_Float16)(x0 - (float)h0), l1 = (_Float16)(x1 - (float)h1);
+                    const int d = 4 * (dq0 + 8 * c) + e, w = 4 * (kp & 3);
+                    *reinterpret_cast<uint32_t *>(vimg + I::v_at(d, kp >> 2) + w) = fl_pack(h0, h1);
+                    *reinterpret_cast<uint32_t *>(vimg + I::v_at(HD + d, kp >> 2) + w) = fl_pack(l0, l1);
                 }
-            ek[j] = fl_exp(fl_pair_max(km));
-            ev[j] = fl_exp(fl_pair_max(vm));
         }
-        if (dq0 == 0) {
-            kex[2 * kp] = ek[0]; kex[2 * kp + 1] = ek[1];
-            vex[2 * kp] = ev[0]; vex[2 * kp + 1] = ev[1];
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                _Float16 hi[4], lo[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float x = __builtin_amdgcn_ldexpf(kr[j][c][e], ek[j]);
-                    hi[e] = (_Float16)x;
-                    lo[e] = (_Float16)(x - (float)hi[e]);
-                }
-                const int dq = dq0 + 8 * c, rk = fl_krow(2 * kp + j);
-                *reinterpret_cast<uint2 *>(img + I::k_at(rk, dq >> 1) + 8 * (dq & 1)) =
-                    make_uint2(fl_pack(hi[0], hi[1]), fl_pack(hi[2], hi[3]));
-                *reinterpret_cast<uint2 *>(img + I::k_at(FL_BK + rk, dq >> 1) + 8 * (dq & 1)) =
-                    make_uint2(fl_pack(lo[0], lo[1]), fl_pack(lo[2], lo[3]));
-            }
-#pragma unroll
-        for (int c = 0; c < NC; c++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float x0 = __builtin_amdgcn_ldexpf(vr[0][c][e], ev[0]);
-                const float x1 = __builtin_amdgcn_ldexpf(vr[1][c][e], ev[1]);
-                const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
-                const _Float16 l0 = (_Float16)(x0 - (float)h0), l1 = (_Float16)(x1 - (float)h1);
-                const int d = 4 * (dq0 + 8 * c) + e, w = 4 * (kp & 3);
-                *reinterpret_cast<uint32_t *>(vimg + I::v_at(d, kp >> 2) + w) = fl_pack(h0, h1);
-                *reinterpret_cast<uint32_t *>(vimg + I::v_at(HD + d, kp >> 2) + w) = fl_pack(l0, l1);
-            }
     }
+};
+
+// grid (kv heads, tiles of the pass's keys [0, pos_base + n_tok))
+template <int HD, bool F16>
+__global__ __launch_bounds__(WG) void k_pf_kvsplit(AttnArgs a) {
+    using I = FlImg<HD, F16>;
+    __shared__ __align__(16) uint8_t img[I::HBYTES];   // the image as it goes to HBM
+    const int tid = threadIdx.x, g = blockIdx.x, kt = blockIdx.y;
+    FlTile<HD, F16> t;
+    t.load(a, g, kt * FL_BK, a.pos_base + a.n_tok - 1, tid);
+    t.image(img, img + I::KE, tid);
     __syncthreads();
     // the image to HBM as it lies
     u32x4 *dst = reinterpret_cast<u32x4 *>(a.kvimg + ((size_t)g * a.kvimg_tiles + kt) * I::HBYTES);
@@ -1137,6 +1148,11 @@ __device__ __forceinline__ void fl_load_lds(const uint8_t *src, uint8_t *dst) {
     __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
 }
 
+#define FL_Q 1
+#define FL_SCORES 2
+#define FL_SOFTMAX 3
+#define FL_PV 4
+#define FL_OUT 5
 // 64 rows per workgroup, two workgroups per CU: one's barriers overlap the
 // other's products (128 rows per workgroup, one per CU, measured slower).
 // Per key tile, with its K part and exponents (kimg) and its V part (vimg)
@@ -1156,6 +1172,7 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
     using I = FlImg<HD, F16>;
     constexpr int NQ = HD / 32;         // 32-dim steps of a score product
     constexpr int ND = HD / 16;         // 16-dim output products
+    constexpr bool KEY0 = KS == 1;
     constexpr int GT = 64 * RW;                          // threads per key-tile group
     constexpr int BR = 16 * RW;                          // rows per workgroup
     constexpr int KE_N = (I::KE_SLABS + RW - 1) / RW, KE_MIN = I::KE_SLABS / RW;   // K-part slabs per wave
@@ -1184,25 +1201,8 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
     int eq;
     {
         const float *qr = a.q + (size_t)b * a.q_stride + (size_t)(g * G + h) * HD + 8 * q;
-        f32x4 qv[NQ][2];
-        float mx = 0.0f;
-#pragma unroll
-        for (int s = 0; s < NQ; s++)
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                qv[s][u] = *reinterpret_cast<const f32x4 *>(qr + 32 * s + 4 * u);
-#pragma unroll
-                for (int e = 0; e < 4; e++) mx = fmaxf(mx, fabsf(qv[s][u][e]));
-            }
-        eq = fl_exp(fl_quarter_max(mx));
-#pragma unroll
-        for (int s = 0; s < NQ; s++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float x = __builtin_amdgcn_ldexpf(qv[s][e >> 2][e & 3], eq);
-                qh[s][e] = (_Float16)x;
-                ql[s][e] = (_Float16)(x - (float)qh[s][e]);
-            }
+#define FL_PIECE FL_Q
+#include "fl_step.inc"
     }
     const float sscale = a.inv_sqrt * 1.4426950408889634f;
     float m = -INFINITY, lsum = 0.0f;
@@ -1250,37 +1250,8 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
         for (int kk = 0; kk < 4; kk++) sc[kk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         int kx[2][8], vx[2][8];   // the per-key exponents of this lane's 16 keys
         if (act) {
-#pragma unroll
-        for (int s = 0; s < NQ; s++) {
-            f16x8 kh[4], kl[4];
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                kh[kk] = *reinterpret_cast<const f16x8 *>(kimg + I::k_at(16 * kk + i, 4 * s + q));
-                if constexpr (!F16) kl[kk] = *reinterpret_cast<const f16x8 *>(kimg + I::k_at(FL_BK + 16 * kk + i, 4 * s + q));
-            }
-            if constexpr (!F16) {
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++) sc[kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[kk], qh[s], sc[kk], 0, 0, 0);
-            }
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) sc[kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[kk], ql[s], sc[kk], 0, 0, 0);
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) sc[kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[kk], qh[s], sc[kk], 0, 0, 0);
-        }
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                if constexpr (F16) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) kx[t][4 * u + e] = vx[t][4 * u + e] = 0;
-                } else {
-                    const int4 ka = *reinterpret_cast<const int4 *>(&kex[32 * t + 8 * q + 4 * u]);
-                    const int4 va = *reinterpret_cast<const int4 *>(&vex[32 * t + 8 * q + 4 * u]);
-                    kx[t][4 * u] = ka.x; kx[t][4 * u + 1] = ka.y; kx[t][4 * u + 2] = ka.z; kx[t][4 * u + 3] = ka.w;
-                    vx[t][4 * u] = va.x; vx[t][4 * u + 1] = va.y; vx[t][4 * u + 2] = va.z; vx[t][4 * u + 3] = va.w;
-                }
-            }
+#define FL_PIECE FL_SCORES
+#include "fl_step.inc"
         }
         if (more) {   // every wave is past its kimg reads: the next tile's K part may land
             fl_sync();
@@ -1288,54 +1259,8 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
         }
         f16x8 ph[2], pl[2];
         if (act) {
-        // running softmax of the row (log2 units); keys past the row's position
-        // are masked (only in tiles that reach past the workgroup's first row)
-        float mx = -INFINITY;
-        int el = 1 << 20;   // the smallest V-row exponent among the row's visible keys of the tile
-        auto scores = [&](auto masked) {
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int t = kk >> 1, jj = 4 * (kk & 1) + r;
-                    float v = __builtin_amdgcn_ldexpf(sc[kk][r], -(eq + kx[t][jj])) * sscale;
-                    if constexpr (decltype(masked)::value) {
-                        const bool vis = k0 + 32 * t + 8 * q + jj <= pos;
-                        v = vis ? v : -INFINITY;
-                        if (vis) el = min(el, vx[t][jj]);
-                    } else {
-                        el = min(el, vx[t][jj]);
-                    }
-                    sc[kk][r] = v;
-                    mx = fmaxf(mx, v);
-                }
-        };
-        if (k0 + FL_BK - 1 <= kfirst) scores(FlMask<false>{});
-        else scores(FlMask<true>{});
-        // finite: key 0 is in the first tile (KS = 2: group 1's first tile can
-        // hide every key from a row; its maximum stays -inf and mz stands in)
-        const float mn = fmaxf(m, fl_quarter_max(mx));
-        const float mz = KS == 1 || mn != -INFINITY ? mn : 0.0f;
-        const float alpha = __builtin_amdgcn_exp2f(m - mz);   // 0 on the first tile (m = -inf)
-        m = mn;
-        lsum *= alpha;
-        int emin = -(int)fl_quarter_max(-(float)el);
-        if (emin == (1 << 20)) emin = ecur;   // no visible key in this tile
-        const float of = __builtin_amdgcn_ldexpf(alpha, emin - ecur);
-        ecur = emin;
-#pragma unroll
-        for (int d = 0; d < ND; d++) o[d] *= of;
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int t = kk >> 1, jj = 4 * (kk & 1) + r;
-                const float p = __builtin_amdgcn_exp2f(sc[kk][r] - mz);   // masked: 2^-inf = 0
-                lsum += p;
-                const float x = __builtin_amdgcn_ldexpf(p, 14 + emin - vx[t][jj]);
-                ph[t][jj] = (_Float16)x;
-                pl[t][jj] = (_Float16)(x - (float)ph[t][jj]);
-            }
+#define FL_PIECE FL_SOFTMAX
+#include "fl_step.inc"
         }
         if (it > 0) {   // this tile's V part, issued before the next tile's K part
             if (gmore) __builtin_amdgcn_s_waitcnt(fl_vmcnt(KE_MIN));
@@ -1344,23 +1269,8 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
         }
         // ---- O''^T += V'^T . P''^T over keys 32t + 8q + jj
         if (act)
-#pragma unroll
-        for (int t = 0; t < 2; t++) {
-            f16x8 vh[ND], vl[ND];
-#pragma unroll
-            for (int d = 0; d < ND; d++) {
-                vh[d] = *reinterpret_cast<const f16x8 *>(vimg + I::v_at(16 * d + i, 4 * t + q));
-                if constexpr (!F16) vl[d] = *reinterpret_cast<const f16x8 *>(vimg + I::v_at(HD + 16 * d + i, 4 * t + q));
-            }
-            if constexpr (!F16) {
-#pragma unroll
-                for (int d = 0; d < ND; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[d], ph[t], o[d], 0, 0, 0);
-            }
-#pragma unroll
-            for (int d = 0; d < ND; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[d], pl[t], o[d], 0, 0, 0);
-#pragma unroll
-            for (int d = 0; d < ND; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[d], ph[t], o[d], 0, 0, 0);
-        }
+#define FL_PIECE FL_PV
+#include "fl_step.inc"
         if (more) {   // the next K part has landed and every wave is past its vimg reads
             __builtin_amdgcn_s_waitcnt(fl_vmcnt(0));
             fl_sync();
@@ -1405,50 +1315,143 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
             for (int r = 0; r < 4; r++) o[d][r] = __builtin_amdgcn_ldexpf(o[d][r], un) * inv;
     }
     const bool live = r0 + wave * 16 + i < nrows;
-    const size_t col = (size_t)(g * G + h) * HD + 4 * q;
-    const size_t row = (size_t)b * a.n_heads * HD;
-    if (live) {
+#define FL_PIECE FL_OUT
+#include "fl_step.inc"
+}
+
+// k_pf_few_attn: the attention of a pass of few rows behind a history (the
+// next turn of a conversation), where k_pf_flash16's grid is a few row tiles
+// that walk every key tile one after the other (8 kv heads x 46 rows at 540
+// keys: 16 workgroups, 17 us per layer, behind 5 us of k_pf_kvsplit).  A
+// workgroup takes 64 rows of a kv head and a range of its key tiles, converts
+// each tile in LDS (fl_tile's image, never written to HBM: at most a few row
+// tiles share it) with the next tile's rows already in flight, and leaves its
+// running softmax to k_pf_few_merge; with one range it finishes the output.
+// part: o [z][n_kv * G][n_tok][HD], then (m, l) as float2 [z][n_kv * G][n_tok].
+template <int HD, bool F16>
+__global__ __launch_bounds__(WG) void k_pf_few_attn(AttnArgs a, int per) {
+    using I = FlImg<HD, F16>;
+    constexpr int NQ = HD / 32, ND = HD / 16;
+    constexpr bool KEY0 = false;
+    __shared__ __align__(16) uint8_t kimg[I::KE], vimg[I::VBYTES];
+    const int *kex = reinterpret_cast<const int *>(kimg + I::KBYTES), *vex = kex + FL_BK;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 15, q = lane >> 4;
+    const int g = blockIdx.x, z = blockIdx.y, r0 = blockIdx.z * FL_BR;
+    const int G = a.n_heads / a.n_kv, nrows = a.n_tok * G;
+    const int R = min(r0 + wave * 16 + i, nrows - 1);   // this lane's row (padding rows repeat the last)
+    const int b = R / G, h = R % G, pos = a.pos_base + b;
+    const int klast = a.pos_base + a.n_tok - 1, kend = a.pos_base + (min(r0 + FL_BR, nrows) - 1) / G;
+    const int kfirst = a.pos_base + r0 / G;
+    const int kt0 = z * per, kt1 = min(kt0 + per, kend / FL_BK + 1);   // this workgroup's tiles
+    FlTile<HD, F16> t;
+    t.load(a, g, kt0 * FL_BK, klast, tid);
+    f16x8 qh[NQ], ql[NQ];
+    int eq;
+    {
+        const float *qr = a.q + (size_t)b * a.q_stride + (size_t)(g * G + h) * HD + 8 * q;
+#define FL_PIECE FL_Q
+#include "fl_step.inc"
+    }
+    const float sscale = a.inv_sqrt * 1.4426950408889634f;
+    float m = -INFINITY, lsum = 0.0f;
+    int ecur = 0;
+    f32x4 o[ND];
+#pragma unroll
+    for (int d = 0; d < ND; d++) o[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const bool busy = r0 + wave * 16 < nrows;   // uniform over the wave
+    for (int kt = kt0; kt < kt1; kt++) {
+        if (kt > kt0) __syncthreads();   // every wave is past the last tile's reads
+        t.image(kimg, vimg, tid);
+        if (kt + 1 < kt1) t.load(a, g, (kt + 1) * FL_BK, klast, tid);
+        __syncthreads();
+        if (!busy) continue;
+        f32x4 sc[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) sc[kk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        int kx[2][8], vx[2][8];
+        f16x8 ph[2], pl[2];
+        const int k0 = kt * FL_BK;
+#define FL_PIECE FL_SCORES
+#include "fl_step.inc"
+#define FL_PIECE FL_SOFTMAX
+#include "fl_step.inc"
+#define FL_PIECE FL_PV
+#include "fl_step.inc"
+    }
+    const bool live = r0 + wave * 16 + i < nrows;
+    const float l = fl_quarter_sum(lsum);
+    const int un = -(14 + ecur);
+    if (gridDim.y == 1) {
+        const float inv = 1.0f / l;
 #pragma unroll
         for (int d = 0; d < ND; d++)
-            *reinterpret_cast<float4 *>(a.out + row + col + 16 * d) = make_float4(o[d][0], o[d][1], o[d][2], o[d][3]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[d][r] = __builtin_amdgcn_ldexpf(o[d][r], un) * inv;
+#define FL_PIECE FL_OUT
+#include "fl_step.inc"
+        return;
     }
+    if (!live) return;
+    const size_t rows = (size_t)a.n_heads * a.n_tok, row = (size_t)z * rows + (size_t)(g * G + h) * a.n_tok + b;
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+        f32x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = __builtin_amdgcn_ldexpf(o[d][r], un);
+        *reinterpret_cast<f32x4 *>(a.part + row * HD + 16 * d + 4 * q) = v;
+    }
+    if (q == 0) reinterpret_cast<float2 *>(a.part + (size_t)gridDim.y * rows * HD)[row] = make_float2(m, l);
+}
+
+// The ranges' softmaxes of each (head, token) row, a wave per row: lane z
+// weighs range z (at most 64), HD / 4 lanes with four dims each add every
+// (256 / HD)-th range's partial, and the output's Q8_0 blocks follow
+// (k_quant_rows's arithmetic).
+template <int HD>
+__global__ __launch_bounds__(WG) void k_pf_few_merge(AttnArgs a, int nz) {
+    constexpr int LPR = HD / 4, NG = 64 / LPR, U = 4;
+    const int rows = a.n_heads * a.n_tok, lane = threadIdx.x & 63, grp = lane / LPR, d0 = 4 * (lane % LPR);
+    const int R = blockIdx.x * NWAVE + (threadIdx.x >> 6), row = min(R, rows - 1);
+    const float *part = a.part + (size_t)row * HD + d0;
+    f32x4 v[U];
+    auto load = [&](int z0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = *reinterpret_cast<const f32x4 *>(part + (size_t)min(z0 + u * NG + grp, nz - 1) * rows * HD);
+    };
+    load(0);
+    const float2 p = reinterpret_cast<const float2 *>(a.part + (size_t)nz * rows * HD)[(size_t)min(lane, nz - 1) * rows + row];
+    const float m = wave_max(p.x);   // finite: some range holds key 0
+    const float w = lane < nz ? __builtin_amdgcn_exp2f(p.x - m) : 0.0f;
+    const float l = wave_sum(p.y * w);
+    f32x4 o{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int z0 = 0; z0 < nz; z0 += U * NG) {
+        if (z0 > 0) load(z0);
+#pragma unroll
+        for (int u = 0; u < U; u++) o += v[u] * __shfl(w, z0 + u * NG + grp);   // past the last range: lanes of weight 0
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        o[e] = xor32_add(o[e]);
+        if (NG == 4) o[e] = xor16_add(o[e]);
+    }
+    o *= 1.0f / l;
+    const float mx = max8(fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), fabsf(o.w))));
+    const float d = mx / 127.0f;
+    const float id = d > 0.0f ? 1.0f / d : 0.0f;
+    int c[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) c[e] = (int)fminf(fmaxf(roundf(o[e] * id), -127.0f), 127.0f);
+    const int cs = sum8(c[0] + c[1] + c[2] + c[3]);
+    if (R >= rows || grp > 0) return;
+    const int head = row / a.n_tok, b = row % a.n_tok;
+    const size_t at = ((size_t)b * a.n_heads + head) * HD + d0;
+    *reinterpret_cast<f32x4 *>(a.out + at) = o;
     if (!a.qx) return;
-    // the output's Q8_0 blocks for wo, with k_quant_rows's arithmetic: block
-    // bk (dims 32bk ..) is o[2bk], o[2bk + 1] of the row's four lanes
-    const int nbk = a.n_heads * HD / QB;
-#pragma unroll
-    for (int bk = 0; bk < ND / 2; bk++) {
-        float mx = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) mx = fmaxf(mx, fabsf(o[2 * bk + u][r]));
-        mx = fl_quarter_max(mx);
-        const float dsc = mx / 127.0f;
-        const float id = dsc > 0.0f ? 1.0f / dsc : 0.0f;
-        int cs = 0;
-        uint32_t pk[2];
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            pk[u] = 0;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int cq = (int)fminf(fmaxf(roundf(o[2 * bk + u][r] * id), -127.0f), 127.0f);
-                cs += cq;
-                pk[u] |= ((uint32_t)cq & 0xffu) << (8 * r);
-            }
-        }
-        cs = (int)fl_quarter_sum((float)cs);   // exact: |sum| <= 32 * 127
-        if (live) {
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-                *reinterpret_cast<uint32_t *>(a.qx + row + col + 16 * (2 * bk + u)) = pk[u];
-            if (q == 0) {
-                const size_t blk = (size_t)b * nbk + ((size_t)(g * G + h) * HD) / QB + bk;
-                a.qdx[blk] = h2f(f2h(dsc));
-                a.qxs[blk] = cs;
-            }
-        }
+    *reinterpret_cast<uint32_t *>(a.qx + at) = ((uint32_t)c[0] & 0xffu) | (((uint32_t)c[1] & 0xffu) << 8) |
+                                               (((uint32_t)c[2] & 0xffu) << 16) | (((uint32_t)c[3] & 0xffu) << 24);
+    if (threadIdx.x % 8 == 0) {
+        a.qdx[at / QB] = h2f(f2h(d));
+        a.qxs[at / QB] = cs;
     }
 }
 
@@ -1458,12 +1461,44 @@ static int env_int_attn(const char *name, int dflt) {
     return v && *v ? atoi(v) : dflt;
 }
 
+// k_pf_few_attn: passes behind a history whose rows are at most FEW_ROW_TILES
+// row tiles
+constexpr int FEW_ROW_TILES = 4, FEW_RANGES = 32;   // (the merge weighs at most 64 ranges)
+bool attn_few_rows(int hd, int G, int pos_base, int n_tok) {
+    return (hd == 64 || hd == 128) && pos_base > 0 && (n_tok * G + FL_BR - 1) / FL_BR <= FEW_ROW_TILES &&
+           env_int_attn("EHIP_PF_FEW", 1);
+}
+// Key ranges: enough for a workgroup per CU, but one (and no merge) for up to
+// two tiles, and no more than a.part holds (a.max_chunks).
+static int launch_few_attn(hipStream_t st, bool f16kv, const AttnArgs &a, int row_tiles) {
+    const int nkt = (a.pos_base + a.n_tok + FL_BK - 1) / FL_BK;
+    int nz = nkt <= 2 || !a.part || a.max_chunks < 1 ? 1 : std::min({nkt, FEW_RANGES, std::max(1, 256 / (a.n_kv * row_tiles)), a.max_chunks});
+    const int per = (nkt + std::max(nz, 1) - 1) / std::max(nz, 1);
+    nz = (nkt + per - 1) / per;
+    const dim3 g(a.n_kv, nz, row_tiles);
+    const dim3 gm((a.n_heads * a.n_tok + NWAVE - 1) / NWAVE);
+#define FA(H, F) hipLaunchKernelGGL((k_pf_few_attn<H, F>), g, dim3(WG), 0, st, a, per);
+    if (a.hd == 64) {
+        if (f16kv) { FA(64, true) } else { FA(64, false) }
+        if (nz > 1) hipLaunchKernelGGL((k_pf_few_merge<64>), gm, dim3(WG), 0, st, a, nz);
+    } else {
+        if (f16kv) { FA(128, true) } else { FA(128, false) }
+        if (nz > 1) hipLaunchKernelGGL((k_pf_few_merge<128>), gm, dim3(WG), 0, st, a, nz);
+    }
+#undef FA
+    return 0;
+}
+
 int launch_attention_mfma(hipStream_t st, bool f16kv, const AttnArgs &a, bool *quantized) {
     if (quantized) *quantized = false;
     if (a.n_kv <= 0 || a.n_heads % a.n_kv != 0 || a.n_tok <= 0 || a.q_stride % 4) return -1;
     if (a.qx && (!a.qdx || !a.qxs)) return -1;
     const int G = a.n_heads / a.n_kv;
     const dim3 grid(a.n_kv, (a.n_tok * G + FL_BR - 1) / FL_BR);
+    if (attn_few_rows(a.hd, G, a.pos_base, a.n_tok)) {
+        if (quantized) *quantized = a.qx != nullptr;
+        return launch_few_attn(st, f16kv, a, (int)grid.y);
+    }
     if (a.hd == 64 || a.hd == 128) {
         const int nkt = (a.pos_base + a.n_tok + FL_BK - 1) / FL_BK;
         if (!a.kvimg || a.kvimg_tiles < nkt) return -1;

@@ -1257,7 +1257,8 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             // fused q|k|v epilogues (EHIP_PF_KVIMG=0 leaves them to
             // k_pf_kvsplit)
             const bool img_ok = !exact && (hd == 64 || hd == 128) && s->pf_kvimg && pos0 % 64 == 0 &&
-                                s->pf_kvimg_tiles >= (pos0 + mt + 63) / 64 && env_int("EHIP_PF_KVIMG", 1);
+                                s->pf_kvimg_tiles >= (pos0 + mt + 63) / 64 &&
+                                !attn_few_rows(hd, c.n_heads / c.n_kv_heads, pos0, mt) && env_int("EHIP_PF_KVIMG", 1);
             if (few) {
                 if (img_ok) {
                     p.kvimg = s->pf_kvimg;
@@ -1297,6 +1298,9 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             at.kvimg = s->pf_kvimg; at.kvimg_tiles = s->pf_kvimg_tiles;
             at.ldk = attn_prefill_ldk(pos0, mt);
             at.kvimg_fused = img_fused ? 1 : 0;
+            // H holds nothing until the w1|w3 product
+            at.part = s->H;
+            at.max_chunks = (int)std::min<size_t>((size_t)s->pf_chunk * 2 * hid / ((size_t)c.n_heads * mt * (hd + 2)), 1 << 20);
             // the attention can quantize its own output for wo (not for F32
             // weights, whose product reads the fp32 rows)
             bool quantized = false;

@@ -80,6 +80,8 @@ struct AttnArgs {
     // decode: chunk partials, o [n_heads][max_chunks][hd], then (m, l)
     // [n_heads][max_chunks], then (with xm_cnt) the launch token of each
     // chunk's partials, int [n_kv][max_chunks]
+    // prefill on matrix cores: partials of at most max_chunks key ranges, o
+    // [max_chunks][n_heads][n_tok][hd], then (m, l) [max_chunks][n_heads][n_tok]
     float *part;
     int max_chunks;
     // decode, optional: merge the chunks of each kv head inside the chunk
@@ -152,6 +154,9 @@ int launch_attention(hipStream_t st, bool f16kv, const AttnArgs &a, bool *quanti
 // matrix cores with split operands for head_dim 64 / 128 (which also write
 // a.qx/qdx/qxs when set, reported in *quantized), fp32 ones for 48
 int launch_attention_mfma(hipStream_t st, bool f16kv, const AttnArgs &a, bool *quantized = nullptr);
+// whether that attention reads the cache itself (a pass of few rows behind a
+// history) and no K/V tile images
+bool attn_few_rows(int hd, int G, int pos_base, int n_tok);
 // bytes of the K/V tile images the matrix-core prefill attention needs for
 // ctx positions (0: head_dim without images)
 size_t attn_kvimg_bytes(int hd, bool f16kv, int ctx, int n_kv);

@@ -1,5 +1,6 @@
-"""Passes of few tokens: their products (gemm_few.hip) against float64 on the
-GPU's own inputs at the edges of their tiles (kernel_check's bounds).
+"""Passes of few tokens: their products (gemm_few.hip), and their attention
+behind a history (k_pf_few_attn, k_pf_few_merge), against float64 on the GPU's
+own inputs at the edges of their tiles (kernel_check's bounds).
 
 The products' sums: K is split over up to 16 waves of at most 16 blocks each,
 so a sum is a chain of at most 16 fmas and one of at most 15 additions, within
@@ -58,3 +59,13 @@ def run(shape, n, kv16, start):
 @pytest.mark.parametrize("shape", list(SHAPES))
 def test_products(shape, n):
     run(shape, n, False, 0)
+
+
+# a history inside the first tile, on a tile's edge, off it, of many key
+# ranges; rows that fill 64-row tiles to the last and past it, up to the four
+# the kernel takes and one more, which it does not
+@pytest.mark.parametrize("shape,n,start,kv16", [("a", 1, 1, False), ("a", 64, 640, True), ("b", 22, 129, False), ("b", 85, 1500, True),
+                                                ("c", 36, 63, True), ("c", 37, 640, False), ("d", 23, 517, True), ("d", 128, 1900, False),
+                                                ("d", 2, 126, False), ("e", 33, 65, True), ("e", 9, 2000, False)])
+def test_attention_behind_a_history(shape, n, start, kv16):
+    run(shape, n, kv16, start)
