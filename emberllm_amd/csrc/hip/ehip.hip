@@ -459,6 +459,9 @@ struct EhipState {
     struct PfGraph { StepGraph sg; int pos0 = -1, n = 0, last = 0; unsigned long long used = 0; };
     PfGraph pfg[PF_GRAPHS];
     unsigned long long pf_clock = 0;
+    // the last PF_GRAPHS pass shapes that ran once, without a graph
+    struct PfShape { int pos0 = -1, n = 0, last = 0; } pf_once[PF_GRAPHS];
+    unsigned pf_once_next = 0;
     StepGraph gen[2];   // device greedy loop: 1 step, GEN_UNROLL steps
     // device sampler: xorshift64* state, history ring, candidates; the
     // sampling decode graph is captured for one parameter set
@@ -1370,32 +1373,35 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
     return 0;
 }
 
-// The graph of a prefill pass shape, captured on first use.
-static hipGraphExec_t prefill_graph(EhipState *s, int pos0, int mt, bool last, int pass) {
+// One prefill pass.  A shape's first pass is launched kernel by kernel and its
+// second captures the graph that it and later ones replay: each turn of a
+// conversation starts at another position, so most shapes run once, and
+// capturing and instantiating their launches (Qwen3-0.6B shape, 170 to 226
+// kernels) takes 0.4-0.6 ms of host time before the first kernel starts,
+// where the launches themselves hide behind the kernels.  Eager as well while
+// a layer's tensors are captured for inspection, or with graphs off.
+static int run_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass) {
+    if (!s->graph_mode || s->pdbg_layer >= 0) return enq_prefill_pass(s, pos0, mt, last, pass);
     EhipState::PfGraph *hit = nullptr, *lru = &s->pfg[0];
     for (auto &pg : s->pfg) {
         if (pg.sg.x && pg.pos0 == pos0 && pg.n == mt && pg.last == (int)last) hit = &pg;
         if (pg.used < lru->used) lru = &pg;
     }
     if (!hit) {
+        bool once = false;
+        for (auto &o : s->pf_once) once |= o.pos0 == pos0 && o.n == mt && o.last == (int)last;
+        if (!once) {
+            s->pf_once[s->pf_once_next++ % PF_GRAPHS] = {pos0, mt, (int)last};
+            return enq_prefill_pass(s, pos0, mt, last, pass);
+        }
         hit = lru;
         graph_free(hit->sg);
-        HCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal), nullptr);
-        const int rc = enq_prefill_pass(s, pos0, mt, last, pass);
-        hipGraph_t g = nullptr;
-        const hipError_t e = hipStreamEndCapture(s->st, &g);
-        if (rc) { if (g) (void)hipGraphDestroy(g); return nullptr; }
-        if (e != hipSuccess) { set_err("hipStreamEndCapture: %s", hipGetErrorString(e)); return nullptr; }
-        hit->sg.g = g;
-        if (hipGraphInstantiate(&hit->sg.x, g, nullptr, nullptr, 0) != hipSuccess) {
-            graph_free(hit->sg);
-            set_err("prefill graph instantiation failed");
-            return nullptr;
-        }
+        if (graph_capture(s, hit->sg, 1, [&]() { return enq_prefill_pass(s, pos0, mt, last, pass); })) return -1;
         hit->pos0 = pos0; hit->n = mt; hit->last = last;
     }
     hit->used = ++s->pf_clock;
-    return hit->sg.x;
+    HCHK(hipGraphLaunch(hit->sg.x, s->st), -1);
+    return 0;
 }
 
 extern "C" float *ehip_prefill(EhipState *s, const int *ids, int n, int start) {
@@ -1408,15 +1414,7 @@ extern "C" float *ehip_prefill(EhipState *s, const int *ids, int n, int start) {
         const int mt = std::min(s->pf_chunk, n - c0), pass = c0 / s->pf_chunk;
         const bool last = c0 + mt == n;
         HCHK(hipMemcpyAsync(s->ids_d, ids + c0, 4 * (size_t)mt, hipMemcpyHostToDevice, s->st), nullptr);
-        // one graph per pass shape; eager launches while a layer's tensors
-        // are being captured for inspection, or with graphs switched off
-        if (s->graph_mode && s->pdbg_layer < 0) {
-            const hipGraphExec_t x = prefill_graph(s, start + c0, mt, last, pass);
-            if (!x) return nullptr;
-            HCHK(hipGraphLaunch(x, s->st), nullptr);
-        } else if (enq_prefill_pass(s, start + c0, mt, last, pass)) {
-            return nullptr;
-        }
+        if (run_prefill_pass(s, start + c0, mt, last, pass)) return nullptr;
     }
     HCHK(hipStreamSynchronize(s->st), nullptr);
     return s->logits_h;
