@@ -1366,8 +1366,9 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             if (rc) { set_err("a prefill kernel could not be launched for this shape"); return -1; }
         }
         if (last) {
-            if (enq_head(s, s->X + (size_t)(mt - 1) * c.dim)) { set_err("head launch failed"); return -1; }
-            HCHK(hipMemcpyAsync(s->logits_h, s->logits_d, 4 * (size_t)c.vocab_size, hipMemcpyDeviceToHost, s->st), -1);
+            MatvecArgs a = head_args(s, s->X + (size_t)(mt - 1) * c.dim);
+            a.out_host = s->logits_h;   // as a decode step's: stored while the head's weights stream
+            if (mv(s, PRO_NORM, EPI_STORE, a)) { set_err("head launch failed"); return -1; }
         }
     }
     return 0;
