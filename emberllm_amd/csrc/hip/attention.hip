@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
     using I = FlImg<HD, F16>;
     constexpr int NQ = HD / 32;         // 32-dim steps of a score product
     constexpr int ND = HD / 16;         // 16-dim output products
-    constexpr bool KEY0 = KS == 1;
+    constexpr bool KEY0 = KS == 1, QK = false;
     constexpr int GT = 64 * RW;                          // threads per key-tile group
     constexpr int BR = 16 * RW;                          // rows per workgroup
     constexpr int KE_N = (I::KE_SLABS + RW - 1) / RW, KE_MIN = I::KE_SLABS / RW;   // K-part slabs per wave
@@ -1319,6 +1319,116 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
 #include "fl_step.inc"
 }
 
+// RMSNorm over a head vector's squares ss (model.c:50-55); RoPE of four
+// dims x from i on (model.c:66-80): neox rotates them with the dims HD / 2 on,
+// interleaved rotates its two pairs.
+__device__ __forceinline__ float fl_rms(float ss, int hd, float eps) { return 1.0f / sqrtf(ss / (float)hd + eps); }
+__device__ __forceinline__ void fl_rope_neox(const float2 *cs, f32x4 &x, f32x4 &y) {
+    const f32x4 a = reinterpret_cast<const f32x4 *>(cs)[0], b = reinterpret_cast<const f32x4 *>(cs)[1];
+    const f32x4 c = {a.x, a.z, b.x, b.z}, s = {a.y, a.w, b.y, b.w};
+    const f32x4 x0 = x;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        x[e] = x0[e] * c[e] - y[e] * s[e];
+        y[e] = x0[e] * s[e] + y[e] * c[e];
+    }
+}
+__device__ __forceinline__ void fl_rope_pairs(const float2 *cs, f32x4 &x) {
+    const f32x4 a = *reinterpret_cast<const f32x4 *>(cs);   // two (cos, sin)
+    x = f32x4{x.x * a.x - x.y * a.y, x.x * a.y + x.y * a.x, x.z * a.z - x.w * a.w, x.z * a.w + x.w * a.z};
+}
+__device__ __forceinline__ float fl_sq(f32x4 v) { return (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w); }
+// a raw Q row's QK-norm and RoPE (its four lanes' dims as FL_Q holds them)
+template <int HD>
+__device__ __forceinline__ void fl_raw_q(const AttnArgs &a, f32x4 (&qv)[HD / 32][2], int pos, int q) {
+    constexpr int NQ = HD / 32;
+    const float2 *cs = a.rope + (size_t)pos * (HD / 2);
+    if (a.q_norm) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int s = 0; s < NQ; s++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) ss += fl_sq(qv[s][u]);
+        const float sc = fl_rms(fl_quarter_sum(ss), HD, a.eps);
+#pragma unroll
+        for (int s = 0; s < NQ; s++)
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                qv[s][u] = qv[s][u] * sc * *reinterpret_cast<const f32x4 *>(a.q_norm + 32 * s + 8 * q + 4 * u);
+    }
+    if (a.rope_style == ROPE_NEOX) {
+#pragma unroll
+        for (int s = 0; s < NQ / 2; s++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) fl_rope_neox(cs + 32 * s + 8 * q + 4 * u, qv[s][u], qv[s + NQ / 2][u]);
+    } else {
+#pragma unroll
+        for (int s = 0; s < NQ; s++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) fl_rope_pairs(cs + (32 * s + 8 * q + 4 * u) / 2, qv[s][u]);
+    }
+}
+// The pass's own keys among a tile's (positions from pos_base on; keys past
+// the last repeat it) from the raw q|k|v rows: QK-norm and RoPE of k, v as it
+// is, rounded as the cache holds them, into t; with store also to the cache.
+template <int HD, bool F16>
+__device__ __forceinline__ void fl_raw_keys(const AttnArgs &a, FlTile<HD, F16> &t, int g, int k0, bool store, int tid) {
+    constexpr int NC = HD / 32;
+    const int kp = 8 * (tid >> 6) + (tid & 7), dq0 = (tid & 63) >> 3;
+    const int klast = a.pos_base + a.n_tok - 1;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int key = k0 + 2 * kp + j, b = max(min(key, klast) - a.pos_base, 0);
+        const float *row = a.q + (size_t)b * a.q_stride + (size_t)a.n_heads * HD + (size_t)g * HD + 4 * dq0;
+        f32x4 x[NC], v[NC];
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            x[c] = *reinterpret_cast<const f32x4 *>(row + 32 * c);
+            v[c] = *reinterpret_cast<const f32x4 *>(row + a.kv_dim + 32 * c);
+        }
+        const float2 *cs = a.rope + (size_t)(a.pos_base + b) * (HD / 2);
+        if (a.q_norm) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NC; c++) ss += fl_sq(x[c]);
+            const float sc = fl_rms(xor32_add(xor16_add(xor8_add(ss))), HD, a.eps);
+#pragma unroll
+            for (int c = 0; c < NC; c++) x[c] = x[c] * sc * *reinterpret_cast<const f32x4 *>(a.k_norm + 4 * dq0 + 32 * c);
+        }
+        if (a.rope_style == ROPE_NEOX) {
+#pragma unroll
+            for (int c = 0; c < NC / 2; c++) fl_rope_neox(cs + 4 * dq0 + 32 * c, x[c], x[c + NC / 2]);
+        } else {
+#pragma unroll
+            for (int c = 0; c < NC; c++) fl_rope_pairs(cs + (4 * dq0 + 32 * c) / 2, x[c]);
+        }
+        if (key < a.pos_base) continue;
+        const bool put = store && key <= klast;
+        const size_t off = (size_t)key * a.kv_dim + (size_t)g * HD + 4 * dq0;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            if constexpr (F16) {
+                auto half4 = [](f32x4 y) {
+                    return make_uint2(fl_pack((_Float16)y.x, (_Float16)y.y), fl_pack((_Float16)y.z, (_Float16)y.w));
+                };
+                t.kr[j][c] = half4(x[c]);
+                t.vr[j][c] = half4(v[c]);
+                if (put) {
+                    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(a.kc) + off + 32 * c) = t.kr[j][c];
+                    *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(a.vc) + off + 32 * c) = t.vr[j][c];
+                }
+            } else {
+                t.kr[j][c] = x[c];
+                t.vr[j][c] = v[c];
+                if (put) {
+                    *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(a.kc) + off + 32 * c) = x[c];
+                    *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(a.vc) + off + 32 * c) = v[c];
+                }
+            }
+        }
+    }
+}
+
 // k_pf_few_attn: the attention of a pass of few rows behind a history (the
 // next turn of a conversation), where k_pf_flash16's grid is a few row tiles
 // that walk every key tile one after the other (8 kv heads x 46 rows at 540
@@ -1328,7 +1438,11 @@ __global__ __launch_bounds__(64 * RW * KS) void k_pf_flash16(AttnArgs a) {
 // tiles share it) with the next tile's rows already in flight, and leaves its
 // running softmax to k_pf_few_merge; with one range it finishes the output.
 // part: o [z][n_kv * G][n_tok][HD], then (m, l) as float2 [z][n_kv * G][n_tok].
-template <int HD, bool F16>
+// QK: a.q holds the product's raw q|k|v rows.  The workgroup takes QK-norm and
+// RoPE of its rows and of the pass's keys in its tiles itself, and the first
+// row tile's workgroups store those keys to the cache, from which only earlier
+// ones are read.
+template <int HD, bool F16, bool QK>
 __global__ __launch_bounds__(WG) void k_pf_few_attn(AttnArgs a, int per) {
     using I = FlImg<HD, F16>;
     constexpr int NQ = HD / 32, ND = HD / 16;
@@ -1340,11 +1454,15 @@ __global__ __launch_bounds__(WG) void k_pf_few_attn(AttnArgs a, int per) {
     const int G = a.n_heads / a.n_kv, nrows = a.n_tok * G;
     const int R = min(r0 + wave * 16 + i, nrows - 1);   // this lane's row (padding rows repeat the last)
     const int b = R / G, h = R % G, pos = a.pos_base + b;
-    const int klast = a.pos_base + a.n_tok - 1, kend = a.pos_base + (min(r0 + FL_BR, nrows) - 1) / G;
+    const int klast = a.pos_base + a.n_tok - 1;
+    // the workgroup's last visible key (the first row tile's go to the last
+    // key, which they store: masked for their rows past those)
+    const int kend = QK && r0 == 0 ? klast : a.pos_base + (min(r0 + FL_BR, nrows) - 1) / G;
     const int kfirst = a.pos_base + r0 / G;
     const int kt0 = z * per, kt1 = min(kt0 + per, kend / FL_BK + 1);   // this workgroup's tiles
     FlTile<HD, F16> t;
-    t.load(a, g, kt0 * FL_BK, klast, tid);
+    const int kread = QK ? a.pos_base - 1 : klast;   // the last key read from the cache
+    if (!QK || kt0 * FL_BK <= kread) t.load(a, g, kt0 * FL_BK, kread, tid);
     f16x8 qh[NQ], ql[NQ];
     int eq;
     {
@@ -1361,8 +1479,10 @@ __global__ __launch_bounds__(WG) void k_pf_few_attn(AttnArgs a, int per) {
     const bool busy = r0 + wave * 16 < nrows;   // uniform over the wave
     for (int kt = kt0; kt < kt1; kt++) {
         if (kt > kt0) __syncthreads();   // every wave is past the last tile's reads
+        if constexpr (QK)
+            if ((kt + 1) * FL_BK > a.pos_base) fl_raw_keys<HD, F16>(a, t, g, kt * FL_BK, r0 == 0, tid);
         t.image(kimg, vimg, tid);
-        if (kt + 1 < kt1) t.load(a, g, (kt + 1) * FL_BK, klast, tid);
+        if (kt + 1 < kt1 && (!QK || (kt + 1) * FL_BK <= kread)) t.load(a, g, (kt + 1) * FL_BK, kread, tid);
         __syncthreads();
         if (!busy) continue;
         f32x4 sc[4];
@@ -1464,20 +1584,22 @@ static int env_int_attn(const char *name, int dflt) {
 // k_pf_few_attn: passes behind a history whose rows are at most FEW_ROW_TILES
 // row tiles
 constexpr int FEW_ROW_TILES = 4, FEW_RANGES = 32;   // (the merge weighs at most 64 ranges)
-bool attn_few_rows(int hd, int G, int pos_base, int n_tok) {
-    return (hd == 64 || hd == 128) && pos_base > 0 && (n_tok * G + FL_BR - 1) / FL_BR <= FEW_ROW_TILES &&
-           env_int_attn("EHIP_PF_FEW", 1);
+bool attn_raw_rows(int hd, int G, int n_tok) {
+    return (hd == 64 || hd == 128) && n_tok > 0 && (n_tok * G + FL_BR - 1) / FL_BR <= FEW_ROW_TILES && env_int_attn("EHIP_PF_FEW", 1);
 }
+bool attn_few_rows(int hd, int G, int pos_base, int n_tok) { return pos_base > 0 && attn_raw_rows(hd, G, n_tok); }
 // Key ranges: enough for a workgroup per CU, but one (and no merge) for up to
 // two tiles, and no more than a.part holds (a.max_chunks).
-static int launch_few_attn(hipStream_t st, bool f16kv, const AttnArgs &a, int row_tiles) {
+static int launch_few_attn(hipStream_t st, bool f16kv, const AttnArgs &a, int row_tiles, bool qk) {
     const int nkt = (a.pos_base + a.n_tok + FL_BK - 1) / FL_BK;
     int nz = nkt <= 2 || !a.part || a.max_chunks < 1 ? 1 : std::min({nkt, FEW_RANGES, std::max(1, 256 / (a.n_kv * row_tiles)), a.max_chunks});
     const int per = (nkt + std::max(nz, 1) - 1) / std::max(nz, 1);
     nz = (nkt + per - 1) / per;
     const dim3 g(a.n_kv, nz, row_tiles);
     const dim3 gm((a.n_heads * a.n_tok + NWAVE - 1) / NWAVE);
-#define FA(H, F) hipLaunchKernelGGL((k_pf_few_attn<H, F>), g, dim3(WG), 0, st, a, per);
+#define FA(H, F)                                                                              \
+    if (qk) hipLaunchKernelGGL((k_pf_few_attn<H, F, true>), g, dim3(WG), 0, st, a, per);      \
+    else hipLaunchKernelGGL((k_pf_few_attn<H, F, false>), g, dim3(WG), 0, st, a, per);
     if (a.hd == 64) {
         if (f16kv) { FA(64, true) } else { FA(64, false) }
         if (nz > 1) hipLaunchKernelGGL((k_pf_few_merge<64>), gm, dim3(WG), 0, st, a, nz);
@@ -1489,6 +1611,14 @@ static int launch_few_attn(hipStream_t st, bool f16kv, const AttnArgs &a, int ro
     return 0;
 }
 
+int launch_attention_raw(hipStream_t st, bool f16kv, const AttnArgs &a, bool *quantized) {
+    if (quantized) *quantized = a.qx != nullptr;
+    if (a.n_kv <= 0 || a.n_heads % a.n_kv != 0 || a.q_stride % 4 || a.kv_dim != a.n_kv * a.hd || (a.qx && (!a.qdx || !a.qxs))) return -1;
+    const int G = a.n_heads / a.n_kv;
+    if (!attn_raw_rows(a.hd, G, a.n_tok)) return -1;
+    return launch_few_attn(st, f16kv, a, (a.n_tok * G + FL_BR - 1) / FL_BR, true);
+}
+
 int launch_attention_mfma(hipStream_t st, bool f16kv, const AttnArgs &a, bool *quantized) {
     if (quantized) *quantized = false;
     if (a.n_kv <= 0 || a.n_heads % a.n_kv != 0 || a.n_tok <= 0 || a.q_stride % 4) return -1;
@@ -1497,7 +1627,7 @@ int launch_attention_mfma(hipStream_t st, bool f16kv, const AttnArgs &a, bool *q
     const dim3 grid(a.n_kv, (a.n_tok * G + FL_BR - 1) / FL_BR);
     if (attn_few_rows(a.hd, G, a.pos_base, a.n_tok)) {
         if (quantized) *quantized = a.qx != nullptr;
-        return launch_few_attn(st, f16kv, a, (int)grid.y);
+        return launch_few_attn(st, f16kv, a, (int)grid.y, false);
     }
     if (a.hd == 64 || a.hd == 128) {
         const int nkt = (a.pos_base + a.n_tok + FL_BK - 1) / FL_BK;

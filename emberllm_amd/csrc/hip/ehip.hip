@@ -1255,6 +1255,13 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             bool exact = s->pf_mode == PF_EXACT;
             if (s->pf_mode == PF_AUTO)
                 exact = s->pf_seq && pos0 + mt <= PF_EXACT_KEYS;
+            // few rows: the attention takes the product's raw rows.  With F32
+            // weights (no QK-norm and RoPE in their product) always; with
+            // quantized ones of 128-dim heads for a single token tile, where a
+            // head per workgroup leaves most CUs without weights to fetch
+            // (Qwen3-0.6B shape, 2 tokens 1059 -> 938 us, 16 tokens 1197 ->
+            // 1107, 32 tokens 1193 -> 1217; 64-dim heads: no gain)
+            const bool raw = !exact && attn_raw_rows(hd, c.n_heads / c.n_kv_heads, mt) && (few ? hd == 128 && mt <= 16 : any_f32);
             bool img_fused = false;   // the q|k|v product wrote the pass's K/V tile images
             // the matrix-core attention's K/V tile images of the pass, in the
             // fused q|k|v epilogues (EHIP_PF_KVIMG=0 leaves them to
@@ -1262,7 +1269,10 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             const bool img_ok = !exact && (hd == 64 || hd == 128) && s->pf_kvimg && pos0 % 64 == 0 &&
                                 s->pf_kvimg_tiles >= (pos0 + mt + 63) / 64 &&
                                 !attn_few_rows(hd, c.n_heads / c.n_kv_heads, pos0, mt) && env_int("EHIP_PF_KVIMG", 1);
-            if (few) {
+            if (raw) {
+                rc |= few ? launch_few_store(s->st, g, NormIn{s->X, y.attn_norm, c.norm_eps}) : launch_gemm(s->st, EPI_STORE, g);
+                if (psnap(DBG_QKV, s->QKV, stride, stride)) return -1;
+            } else if (few) {
                 if (img_ok) {
                     p.kvimg = s->pf_kvimg;
                     p.kvimg_tiles = s->pf_kvimg_tiles;
@@ -1309,7 +1319,8 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             bool quantized = false;
             if (!any_f32) { at.qx = s->qx; at.qdx = s->dxp; at.qxs = s->xsum; }
             rc |= exact ? launch_attention(s->st, s->f16kv, at, &quantized)
-                        : launch_attention_mfma(s->st, s->f16kv, at, &quantized);
+                : raw ? launch_attention_raw(s->st, s->f16kv, at, &quantized)
+                      : launch_attention_mfma(s->st, s->f16kv, at, &quantized);
             if (psnap(DBG_O, s->O, qd, qd)) return -1;
             GemmArgs g2{};
             g2.W = y.wo; g2.units = c.dim; g2.n = mt; g2.qx = s->qx; g2.dx = s->dxp; g2.xs = s->xsum;

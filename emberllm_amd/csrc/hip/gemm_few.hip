@@ -314,6 +314,39 @@ __global__ __launch_bounds__(64 * FEW_NW) void k_few_qkv(GemmArgs a, NormIn in, 
     qkv_finish<HD, F16, FEW_NW, 64 * FEW_NW>(p, hs, exs, nwv, cs, vh, t0, a.n, wave, lane, true);
 }
 
+// out = W . x (+ bias): 16-row tiles, eight waves over K, two of the rows per
+// wave to normalize.
+constexpr int FEW_SW = 8;
+template <int DT>
+__global__ __launch_bounds__(64 * FEW_SW) void k_few_store(GemmArgs a, NormIn in) {
+    constexpr int NCK = FEW_K / (32 * FEW_CB) / FEW_SW, NR = FEW_T / FEW_SW;
+    __shared__ FewRows x;
+    __shared__ __align__(16) uint8_t wbuf[FEW_SW][FewChunk<DT>::BYTES];
+    __shared__ f32x4 red[FEW_SW][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, fg = lane >> 4;
+    const int u0 = blockIdx.x * 16, t0 = blockIdx.y * FEW_T;
+    const int K = a.W.cols, nb = K / QB, nc = (nb + FEW_CB - 1) / FEW_CB, c0 = wave * NCK;
+    FewRow row[NR];
+#pragma unroll
+    for (int j = 0; j < NR; j++) few_row_load(row[j], in, K, min(t0 + wave + FEW_SW * j, a.n - 1), lane);
+    FewWeights<DT, NCK> w;
+    w.load(a.W, u0, c0, nc, lane);
+    f32x4 bias{0.0f, 0.0f, 0.0f, 0.0f};
+    if (a.bias && wave == 0) bias = *reinterpret_cast<const f32x4 *>(a.bias + u0 + 4 * fg);
+#pragma unroll
+    for (int j = 0; j < NR; j++) {
+        const int t = wave + FEW_SW * j;
+        if (t0 + t < a.n) few_row_quant<DT>(row[j], in.eps, K, lane, x.q[t], x.d[t], x.s[t]);
+    }
+    __syncthreads();
+    red[wave][lane] = few_product<DT, NCK>(w, x, c0, nc, nb, wbuf[wave], lane);
+    __syncthreads();
+    if (wave > 0) return;
+    f32x4 acc = red[0][lane];
+    for (int p = 1; p * NCK < nc; p++) acc += red[p][lane];
+    if (t0 + fr < a.n) *reinterpret_cast<f32x4 *>(a.out + (size_t)(t0 + fr) * a.out_stride + u0 + 4 * fg) = a.bias ? acc + bias : acc;
+}
+
 // w1|w3 with the SwiGLU and its Q8_0 rows in the epilogue (swiglu_rows): 32
 // hidden units per workgroup, four row tiles (gate, gate, up, up), four waves
 // each over K.
@@ -399,6 +432,14 @@ int launch_few_qkv(hipStream_t st, bool f16kv, const GemmArgs &a, const NormIn &
     FQ(DT_Q8, 64) FQ(DT_Q8, 128) FQ(DT_Q4, 64) FQ(DT_Q4, 128)
 #undef FQ
     return -1;
+}
+
+int launch_few_store(hipStream_t st, const GemmArgs &a, const NormIn &in) {
+    if (!few_quantized(a.W) || a.W.cols > FEW_K || a.n <= 0 || a.units % 16 != 0 || a.out_stride % 4 != 0) return -1;
+    const dim3 g(a.units / 16, (a.n + FEW_T - 1) / FEW_T), b(64 * FEW_SW);
+    if (a.W.dtype == DT_Q8) hipLaunchKernelGGL((k_few_store<DT_Q8>), g, b, 0, st, a, in);
+    else hipLaunchKernelGGL((k_few_store<DT_Q4>), g, b, 0, st, a, in);
+    return 0;
 }
 
 int launch_few_swiglu(hipStream_t st, const GemmArgs &a, const NormIn &in) {

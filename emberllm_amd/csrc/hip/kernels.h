@@ -157,6 +157,10 @@ int launch_attention_mfma(hipStream_t st, bool f16kv, const AttnArgs &a, bool *q
 // whether that attention reads the cache itself (a pass of few rows behind a
 // history) and no K/V tile images
 bool attn_few_rows(int hd, int G, int pos_base, int n_tok);
+// The attention of a pass of few rows (attn_raw_rows) on the product's raw
+// q|k|v rows (a.q): QK-norm, RoPE and the KV store inside; -1 for others.
+bool attn_raw_rows(int hd, int G, int n_tok);
+int launch_attention_raw(hipStream_t st, bool f16kv, const AttnArgs &a, bool *quantized = nullptr);
 // bytes of the K/V tile images the matrix-core prefill attention needs for
 // ctx positions (0: head_dim without images)
 size_t attn_kvimg_bytes(int hd, bool f16kv, int ctx, int n_kv);
@@ -295,6 +299,8 @@ struct NormIn { const float *x; const float *norm_w; float eps; };   // x: [n][W
 struct FewShape { DMat qkv, wo, w13, w2; int hd, n; };
 bool gemm_few_fits(const FewShape &s);
 int launch_few_qkv(hipStream_t st, bool f16kv, const GemmArgs &a, const NormIn &in, const QkPostArgs &p, float *raw);
+// the q|k|v product alone, on 16-row tiles
+int launch_few_store(hipStream_t st, const GemmArgs &a, const NormIn &in);
 int launch_few_swiglu(hipStream_t st, const GemmArgs &a, const NormIn &in);
 int launch_few_resid(hipStream_t st, const GemmArgs &a);   // EPI_RESID over rows quantized before
 

@@ -104,3 +104,30 @@ def test_decode_products(shape):
     eng.close()
     print(rep, flush=True)
     assert rep.ok, str(rep)
+
+
+# the attention on the product's raw rows: a fresh pass of one and of four
+# row tiles, one behind a history, with interleaved and neox RoPE
+@pytest.mark.parametrize("kv16", [False, True])
+@pytest.mark.parametrize("hd,n,start", [(64, 5, 0), (64, 128, 0), (64, 33, 300), (128, 70, 0), (128, 3, 61)])
+def test_attention_on_raw_rows(hd, n, start, kv16):
+    cfg = dict(configs.TINY["t_f32"], dim=256, hidden_dim=1056, n_heads=4, n_kv_heads=2, head_dim=hd, max_seq_len=1024,
+               qk_norm=int(hd == 128), rope_style=_native.ROPE_NEOX if hd == 128 else _native.ROPE_INTERLEAVED)
+    path = configs.model_path(f"f32w_raw{hd}", cfg)
+    mf = kc.ModelFile(path)
+    ids = np.random.default_rng(n).integers(0, mf.V, start + n)
+    eng = emberllm.Engine(path, ctx=1024, kv_fp16=kv16)
+    if start:
+        eng.prefill(ids[:start])
+    eng.debug_capture_prefill(1, 0)
+    eng.prefill(ids[start:], start=start)
+    qkv, o = (np.asarray(eng.debug_read_prefill(s)[0], dtype=np.float32) for s in (1, 2))
+    k, v = (kc.cache_rows(eng.kv_read(w, 1, start + n), mf, kv16) for w in (0, 1))
+    eng.debug_capture_prefill(-1, 0)
+    eng.close()
+    rep = kc.Report(f"raw rows, hd {hd}, n {n} at {start} kv16={kv16}")
+    pos = start + np.arange(n)
+    kc.check_kv_rows(rep, "kv store", mf, 1, qkv, pos, k, v, kv16)
+    kc.check_attention(rep, "attention", mf, 1, qkv, pos, k, v, o)
+    print(rep, flush=True)
+    assert rep.ok, str(rep)

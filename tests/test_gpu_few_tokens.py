@@ -66,6 +66,7 @@ def test_products(shape, n):
 # the kernel takes and one more, which it does not
 @pytest.mark.parametrize("shape,n,start,kv16", [("a", 1, 1, False), ("a", 64, 640, True), ("b", 22, 129, False), ("b", 85, 1500, True),
                                                 ("c", 36, 63, True), ("c", 37, 640, False), ("d", 23, 517, True), ("d", 128, 1900, False),
-                                                ("d", 2, 126, False), ("e", 33, 65, True), ("e", 9, 2000, False)])
+                                                ("d", 2, 126, False), ("d", 16, 250, True), ("d", 1, 63, False), ("d", 9, 64, True),
+                                                ("e", 33, 65, True), ("e", 9, 2000, False)])
 def test_attention_behind_a_history(shape, n, start, kv16):
     run(shape, n, kv16, start)
