@@ -30,7 +30,7 @@
 
 namespace ehip {
 
-constexpr int FEW_T = 16;              // tokens per workgroup
+constexpr int FEW_T = 16;              // tokens per tile; a workgroup takes TN tiles
 constexpr int FEW_CB = 4;              // quant blocks per chunk (a wave's unit of K)
 constexpr int FEW_NW = 16;             // waves per workgroup
 constexpr int FEW_K = 1024;            // inputs at most of a product that normalizes its rows
@@ -43,7 +43,6 @@ template <int DT> struct FewChunk {
     static constexpr int PITCH = ROW + 16;                 // LDS row pitch
     static constexpr int BYTES = 16 * PITCH;
 };
-constexpr int FEW_XCHUNK = 16 * (FEW_CB * 32 + 16);        // LDS bytes of 16 tokens' codes of a chunk
 
 // Orders a wave's LDS stores before its own later reads of other lanes' data
 // (the LDS executes a wave's instructions in order; this keeps the compiler's
@@ -80,12 +79,12 @@ template <int DT, int NCK> struct FewWeights {
 };
 
 // One chunk: its weights through the wave's LDS buffer, then four blocks into
-// acc.  xp(kb): this lane's eight codes of block kb (token l % 16); sx: the
-// scale bits of the lane's token and block l / 16 (0 where there is no such
-// block); xsum(kb): the code sum (Q4_0).
-template <int DT, class XP, class XS>
-__device__ __forceinline__ void few_chunk(f32x4 &acc, const i32x4 (&wq)[FewChunk<DT>::NL], uint16_t dw, uint8_t *wbuf,
-                                          XP xp, uint16_t sx, XS xsum, int lane) {
+// acc.  xp(n, kb): this lane's eight codes of block kb (token l % 16 of tile
+// n); sx: the scale bits of those tokens and block l / 16 (0 where there is no
+// such block); xsum(n, kb): the code sum (Q4_0).
+template <int DT, int TN, class XP, class XS>
+__device__ __forceinline__ void few_chunk(f32x4 (&acc)[TN], const i32x4 (&wq)[FewChunk<DT>::NL], uint16_t dw, uint8_t *wbuf,
+                                          XP xp, const uint16_t (&sx)[TN], XS xsum, int lane) {
     using C = FewChunk<DT>;
     constexpr int LPR = C::ROW / 16;
     const int fr = lane & 15, fg = lane >> 4;
@@ -93,8 +92,7 @@ __device__ __forceinline__ void few_chunk(f32x4 &acc, const i32x4 (&wq)[FewChunk
     for (int i = 0; i < C::NL; i++)
         *reinterpret_cast<i32x4 *>(wbuf + (lane / LPR + i * (64 / LPR)) * C::PITCH + (lane % LPR) * 16) = wq[i];
     wave_lds_fence();
-    long af[FEW_CB], bf[FEW_CB];
-    int xs[FEW_CB];
+    long af[FEW_CB];
 #pragma unroll
     for (int kb = 0; kb < FEW_CB; kb++) {
         const uint8_t *wp = wbuf + fr * C::PITCH + kb * C::WB;
@@ -104,25 +102,33 @@ __device__ __forceinline__ void few_chunk(f32x4 &acc, const i32x4 (&wq)[FewChunk
             const unsigned long long raw = *reinterpret_cast<const unsigned long long *>(wp + 8 * (fg & 1));
             af[kb] = (long)((raw >> (4 * (fg >> 1))) & 0x0f0f0f0f0f0f0f0full);
         }
-        bf[kb] = xp(kb);
-        xs[kb] = DT == DT_Q4 ? xsum(kb) : 0;
     }
     // A: every lane's scale at k = 4 (l / 16); B: only block kb's lanes, so the
     // product of row i and token j is dw[i][kb] * dx[j][kb]
     f16x4 sa{}, sb{};
     sa[0] = __builtin_bit_cast(_Float16, dw);
-    i32x4 d[FEW_CB];
 #pragma unroll
-    for (int kb = 0; kb < FEW_CB; kb++)
-        d[kb] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[kb], bf[kb], i32x4{0, 0, 0, 0}, 0, 0, 0);
+    for (int n = 0; n < TN; n++) {
+        long bf[FEW_CB];
+        int xs[FEW_CB];
 #pragma unroll
-    for (int kb = 0; kb < FEW_CB; kb++) {
-        sb[0] = __builtin_bit_cast(_Float16, (uint16_t)(fg == kb ? sx : 0));
-        const f32x4 sc = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, sb, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        for (int kb = 0; kb < FEW_CB; kb++) {
+            bf[kb] = xp(n, kb);
+            xs[kb] = DT == DT_Q4 ? xsum(n, kb) : 0;
+        }
+        i32x4 d[FEW_CB];
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int isum = DT == DT_Q4 ? d[kb][r] - 8 * xs[kb] : d[kb][r];
-            acc[r] = fmaf((float)isum, sc[r], acc[r]);
+        for (int kb = 0; kb < FEW_CB; kb++)
+            d[kb] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[kb], bf[kb], i32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+        for (int kb = 0; kb < FEW_CB; kb++) {
+            sb[0] = __builtin_bit_cast(_Float16, (uint16_t)(fg == kb ? sx[n] : 0));
+            const f32x4 sc = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, sb, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int isum = DT == DT_Q4 ? d[kb][r] - 8 * xs[kb] : d[kb][r];
+                acc[n][r] = fmaf((float)isum, sc[r], acc[n][r]);
+            }
         }
     }
     wave_lds_fence();   // the next chunk's stores stay behind these reads
@@ -132,58 +138,67 @@ __device__ __forceinline__ void few_chunk(f32x4 &acc, const i32x4 (&wq)[FewChunk
 // out[token][row] += W . x over rows quantized before (grid: 16-row tiles,
 // 16-token tiles).  Wave w takes chunks w NCK .. of K; each also loads its own
 // part of the tokens' codes.
-template <int DT, int NCK>
+template <int DT, int NCK, int TN>
 __global__ __launch_bounds__(64 * FEW_NW) void k_few_resid(GemmArgs a) {
     using C = FewChunk<DT>;
+    constexpr int XP = FEW_CB * 32 + 16;   // LDS pitch of a token's codes of a chunk
     __shared__ __align__(16) uint8_t wbuf[FEW_NW][C::BYTES];
-    __shared__ __align__(16) uint8_t xbuf[FEW_NW][FEW_XCHUNK];
-    __shared__ f32x4 red[FEW_NW][64];
+    __shared__ __align__(16) uint8_t xbuf[FEW_NW][TN * FEW_T * XP];
+    __shared__ f32x4 red[FEW_NW][TN][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, fg = lane >> 4;
-    const int u0 = blockIdx.x * 16, t0 = blockIdx.y * FEW_T;
+    const int u0 = blockIdx.x * 16, t0 = blockIdx.y * (TN * FEW_T);
     const int K = a.W.cols, nb = K / QB, nc = (nb + FEW_CB - 1) / FEW_CB;
     const int c0 = wave * NCK;
     FewWeights<DT, NCK> w;
-    i32x4 xq[NCK][2];
-    float dx[NCK];
-    int xs[NCK];
-    // the outputs' old values, for the wave that stores them
-    const int to = t0 + fr;
+    i32x4 xq[NCK][2 * TN];
+    float dx[NCK][TN];
+    int xs[NCK][TN];
+    // the outputs' old values, for the waves that store them (wave n tile n)
+    const int to = t0 + FEW_T * min(wave, TN - 1) + fr;
     f32x4 *const op = reinterpret_cast<f32x4 *>(a.out + (size_t)min(to, a.n - 1) * a.out_stride + u0 + 4 * fg);
-    const f32x4 pre = wave == 0 ? *op : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const f32x4 pre = wave < TN ? *op : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int c = 0; c < NCK; c++) {
         const int b0 = (c0 + c) * FEW_CB;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < 2 * TN; i++) {
             const int t = min(t0 + (lane >> 3) + 8 * i, a.n - 1), pb = (lane & 7) * 16;
             xq[c][i] = *reinterpret_cast<const i32x4 *>(a.qx + (size_t)t * K + (size_t)min(b0 + pb / 32, nb - 1) * 32 + pb % 32);
         }
-        const size_t so = (size_t)min(to, a.n - 1) * nb + min(b0 + fg, nb - 1);
-        dx[c] = a.dx[so];
-        xs[c] = DT == DT_Q4 ? a.xs[so] : 0;
+#pragma unroll
+        for (int n = 0; n < TN; n++) {
+            const size_t so = (size_t)min(t0 + FEW_T * n + fr, a.n - 1) * nb + min(b0 + fg, nb - 1);
+            dx[c][n] = a.dx[so];
+            xs[c][n] = DT == DT_Q4 ? a.xs[so] : 0;
+        }
     }
     w.load(a.W, u0, c0, nc, lane);
-    f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 acc[TN] = {};
     uint8_t *xb = xbuf[wave];
     if (c0 < nc) {
 #pragma unroll
         for (int c = 0; c < NCK; c++) {
 #pragma unroll
-            for (int i = 0; i < 2; i++)
-                *reinterpret_cast<i32x4 *>(xb + ((lane >> 3) + 8 * i) * (FEW_CB * 32 + 16) + (lane & 7) * 16) = xq[c][i];
+            for (int i = 0; i < 2 * TN; i++)
+                *reinterpret_cast<i32x4 *>(xb + ((lane >> 3) + 8 * i) * XP + (lane & 7) * 16) = xq[c][i];
             const bool have = (c0 + c) * FEW_CB + fg < nb;
-            few_chunk<DT>(
+            uint16_t sx[TN];
+#pragma unroll
+            for (int n = 0; n < TN; n++) sx[n] = have ? f2h(dx[c][n]) : (uint16_t)0;
+            few_chunk<DT, TN>(
                 acc, w.q[c], w.d[c], wbuf[wave],
-                [&](int kb) { return *reinterpret_cast<const long *>(xb + fr * (FEW_CB * 32 + 16) + kb * 32 + 8 * fg); },
-                have ? f2h(dx[c]) : (uint16_t)0, [&](int kb) { return __shfl(xs[c], fr + 16 * kb); }, lane);
+                [&](int n, int kb) { return *reinterpret_cast<const long *>(xb + (FEW_T * n + fr) * XP + kb * 32 + 8 * fg); },
+                sx, [&](int n, int kb) { return __shfl(xs[c][n], fr + 16 * kb); }, lane);
         }
     }
-    red[wave][lane] = acc;
+#pragma unroll
+    for (int n = 0; n < TN; n++) red[wave][n][lane] = acc[n];
     __syncthreads();
-    if (wave > 0) return;
+    if (wave >= TN) return;
     const int np = (nc + NCK - 1) / NCK;   // waves with a part of K
-    for (int p = 1; p < np; p++) acc += red[p][lane];
-    if (to < a.n) *op = pre + acc;
+    f32x4 v = red[0][wave][lane];
+    for (int p = 1; p < np; p++) v += red[p][wave][lane];
+    if (to < a.n) *op = pre + v;
 }
 
 // ------------------------------------------------- normalized products --
@@ -245,28 +260,31 @@ __device__ __forceinline__ void few_row_quant(const FewRow &r, float eps, int K,
     }
 }
 
-struct FewRows {   // the workgroup's quantized rows, in LDS
-    __align__(16) uint8_t q[FEW_T][FEW_XP];
-    uint16_t d[FEW_T][FEW_K / QB + 2];
-    int s[FEW_T][FEW_K / QB + 1];
+template <int TN> struct FewRows {   // the workgroup's quantized rows, in LDS
+    __align__(16) uint8_t q[TN * FEW_T][FEW_XP];
+    uint16_t d[TN * FEW_T][FEW_K / QB + 2];
+    int s[TN * FEW_T][FEW_K / QB + 1];
 };
 
-// A wave's sum over chunks c0 .. c0 + NCK - 1 (below nc) of its 16 rows.
-template <int DT, int NCK>
-__device__ __forceinline__ f32x4 few_product(const FewWeights<DT, NCK> &w, const FewRows &x, int c0, int nc, int nb,
-                                             uint8_t *wbuf, int lane) {
+// A wave's sums over chunks c0 .. c0 + NCK - 1 (below nc) of its 16 rows.
+template <int DT, int NCK, int TN>
+__device__ __forceinline__ void few_product(f32x4 (&acc)[TN], const FewWeights<DT, NCK> &w, const FewRows<TN> &x, int c0, int nc,
+                                            int nb, uint8_t *wbuf, int lane) {
     const int fr = lane & 15, fg = lane >> 4;
-    f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int n = 0; n < TN; n++) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int c = 0; c < NCK; c++) {
         if (c0 + c >= nc) break;   // uniform over the wave
         const int b0 = (c0 + c) * FEW_CB, sb = b0 + fg;
-        few_chunk<DT>(
+        uint16_t sx[TN];
+#pragma unroll
+        for (int n = 0; n < TN; n++) sx[n] = sb < nb ? x.d[FEW_T * n + fr][sb] : (uint16_t)0;
+        few_chunk<DT, TN>(
             acc, w.q[c], w.d[c], wbuf,
-            [&](int kb) { return *reinterpret_cast<const long *>(x.q[fr] + (size_t)min(b0 + kb, nb - 1) * 32 + 8 * fg); },
-            sb < nb ? x.d[fr][sb] : (uint16_t)0, [&](int kb) { return x.s[fr][min(b0 + kb, nb - 1)]; }, lane);
+            [&](int n, int kb) { return *reinterpret_cast<const long *>(x.q[FEW_T * n + fr] + (size_t)min(b0 + kb, nb - 1) * 32 + 8 * fg); },
+            sx, [&](int n, int kb) { return x.s[FEW_T * n + fr][min(b0 + kb, nb - 1)]; }, lane);
     }
-    return acc;
 }
 
 // q|k|v with k_qkpost's work in the epilogue (qkv_finish): a head vector per
@@ -275,7 +293,7 @@ __device__ __forceinline__ f32x4 few_product(const FewWeights<DT, NCK> &w, const
 template <int DT, int HD, bool F16>
 __global__ __launch_bounds__(64 * FEW_NW) void k_few_qkv(GemmArgs a, NormIn in, QkPostArgs p, float *raw) {
     constexpr int NT = HD / 16, NP = FEW_NW / NT, NCK = FEW_K / (32 * FEW_CB) / NP;   // row tiles, K parts, chunks
-    __shared__ FewRows x;
+    __shared__ FewRows<1> x;
     __shared__ __align__(16) uint8_t wbuf[FEW_NW][FewChunk<DT>::BYTES];
     __shared__ f32x4 red[NP - 1][NT][64];
     __shared__ float hs[QV_T][HD + 1];
@@ -296,7 +314,9 @@ __global__ __launch_bounds__(64 * FEW_NW) void k_few_qkv(GemmArgs a, NormIn in, 
     for (int r = 0; r < 4; r++) bias[r] = a.bias ? a.bias[u0 + 4 * fg + r] : 0.0f;
     if (t0 + wave < a.n) few_row_quant<DT>(row, in.eps, K, lane, x.q[wave], x.d[wave], x.s[wave]);
     __syncthreads();
-    f32x4 acc = few_product<DT, NCK>(w, x, c0, nc, nb, wbuf[wave], lane);
+    f32x4 accs[1];
+    few_product<DT, NCK, 1>(accs, w, x, c0, nc, nb, wbuf[wave], lane);
+    f32x4 acc = accs[0];
     if (part > 0) red[part - 1][tile][lane] = acc;
     __syncthreads();
     if (part == 0) {
@@ -320,7 +340,7 @@ constexpr int FEW_SW = 8;
 template <int DT>
 __global__ __launch_bounds__(64 * FEW_SW) void k_few_store(GemmArgs a, NormIn in) {
     constexpr int NCK = FEW_K / (32 * FEW_CB) / FEW_SW, NR = FEW_T / FEW_SW;
-    __shared__ FewRows x;
+    __shared__ FewRows<1> x;
     __shared__ __align__(16) uint8_t wbuf[FEW_SW][FewChunk<DT>::BYTES];
     __shared__ f32x4 red[FEW_SW][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, fg = lane >> 4;
@@ -339,7 +359,9 @@ __global__ __launch_bounds__(64 * FEW_SW) void k_few_store(GemmArgs a, NormIn in
         if (t0 + t < a.n) few_row_quant<DT>(row[j], in.eps, K, lane, x.q[t], x.d[t], x.s[t]);
     }
     __syncthreads();
-    red[wave][lane] = few_product<DT, NCK>(w, x, c0, nc, nb, wbuf[wave], lane);
+    f32x4 accs[1];
+    few_product<DT, NCK, 1>(accs, w, x, c0, nc, nb, wbuf[wave], lane);
+    red[wave][lane] = accs[0];
     __syncthreads();
     if (wave > 0) return;
     f32x4 acc = red[0][lane];
@@ -350,41 +372,55 @@ __global__ __launch_bounds__(64 * FEW_SW) void k_few_store(GemmArgs a, NormIn in
 // w1|w3 with the SwiGLU and its Q8_0 rows in the epilogue (swiglu_rows): 32
 // hidden units per workgroup, four row tiles (gate, gate, up, up), four waves
 // each over K.
-template <int DT>
+template <int DT, int TN>
 __global__ __launch_bounds__(64 * FEW_NW) void k_few_swiglu(GemmArgs a, NormIn in) {
     constexpr int NT = 2 * SW_U / 16, NP = FEW_NW / NT, NCK = FEW_K / (32 * FEW_CB) / NP;
-    __shared__ FewRows x;
+    static_assert(SW_T == FEW_T, "tokens per tile");
+    __shared__ FewRows<TN> x;
     __shared__ __align__(16) uint8_t wbuf[FEW_NW][FewChunk<DT>::BYTES];
-    __shared__ f32x4 red[NP - 1][NT][64];
-    __shared__ float hs[SW_T][2 * SW_U + 1];
+    __shared__ f32x4 red[NP - 1][NT][TN][64];
+    __shared__ float hs[TN][SW_T][2 * SW_U + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, fg = lane >> 4;
     const int tile = wave % NT, part = wave / NT;
-    const int u0 = blockIdx.x * SW_U, t0 = blockIdx.y * SW_T;
+    const int u0 = blockIdx.x * SW_U, t0 = blockIdx.y * (TN * SW_T);
     const int K = a.W.cols, nb = K / QB, nc = (nb + FEW_CB - 1) / FEW_CB, c0 = part * NCK;
     const int half = tile >> 1, ut = (tile & 1) * 16;   // up rows or gate rows, first unit of the tile
-    FewRow row;
-    few_row_load(row, in, K, min(t0 + wave, a.n - 1), lane);
+    FewRow row[TN];
+#pragma unroll
+    for (int n = 0; n < TN; n++) few_row_load(row[n], in, K, min(t0 + FEW_NW * n + wave, a.n - 1), lane);
     FewWeights<DT, NCK> w;
     w.load(a.W, half * a.pair_off + u0 + ut, c0, nc, lane);
-    if (t0 + wave < a.n) few_row_quant<DT>(row, in.eps, K, lane, x.q[wave], x.d[wave], x.s[wave]);
+#pragma unroll
+    for (int n = 0; n < TN; n++) {
+        const int t = FEW_NW * n + wave;
+        if (t0 + t < a.n) few_row_quant<DT>(row[n], in.eps, K, lane, x.q[t], x.d[t], x.s[t]);
+    }
     __syncthreads();
-    f32x4 acc = few_product<DT, NCK>(w, x, c0, nc, nb, wbuf[wave], lane);
-    if (part > 0) red[part - 1][tile][lane] = acc;
+    f32x4 acc[TN];
+    few_product<DT, NCK, TN>(acc, w, x, c0, nc, nb, wbuf[wave], lane);
+#pragma unroll
+    for (int n = 0; n < TN; n++)
+        if (part > 0) red[part - 1][tile][n][lane] = acc[n];
     __syncthreads();
     if (part == 0) {
 #pragma unroll
-        for (int s = 0; s < NP - 1; s++)
-            if ((s + 1) * NCK < nc) acc += red[s][tile][lane];
+        for (int n = 0; n < TN; n++) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            hs[fr][half * SW_U + ut + 4 * fg + r] = acc[r];
-            if (a.out && t0 + fr < a.n)   // the gate | up products themselves, where asked for
-                a.out[(size_t)(t0 + fr) * a.out_stride + half * a.pair_off + u0 + ut + 4 * fg + r] = acc[r];
+            for (int s = 0; s < NP - 1; s++)
+                if ((s + 1) * NCK < nc) acc[n] += red[s][tile][n][lane];
+            const int t = t0 + SW_T * n + fr;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                hs[n][fr][half * SW_U + ut + 4 * fg + r] = acc[n][r];
+                if (a.out && t < a.n)   // the gate | up products themselves, where asked for
+                    a.out[(size_t)t * a.out_stride + half * a.pair_off + u0 + ut + 4 * fg + r] = acc[n][r];
+            }
         }
     }
     __syncthreads();
-    if (threadIdx.x >= SW_T * 8) return;
-    swiglu_rows(a, hs, u0, t0, threadIdx.x);
+    if (threadIdx.x >= TN * SW_T * 8) return;
+    const int n = threadIdx.x / (SW_T * 8);
+    swiglu_rows(a, hs[n], u0, t0 + SW_T * n, threadIdx.x % (SW_T * 8));
 }
 
 // -------------------------------------------------------------- launches --
@@ -405,17 +441,29 @@ bool gemm_few_fits(const FewShape &s) {
     return s.wo.cols <= most && s.w2.cols <= most;
 }
 
+// Two token tiles per workgroup, whose weights and LDS trips then serve 32
+// tokens, once single tiles give more workgroups than fit the GPU's CUs `per`
+// to a CU at a time, or more than one per CU where the pairs still fit:
+// Qwen3-0.6B shape 64 tokens 1343 -> 1269 us, SmolLM2-135M 128 tokens 1085 ->
+// 961, stories110M 128 tokens 535 -> 477 (below that line the halved grid
+// loses: Qwen2.5-0.5B, w1|w3 456 workgroups at 48 tokens, 355 -> 373).
+static bool few_two(int tiles, int n, int per) {
+    const long g1 = (long)tiles * ((n + FEW_T - 1) / FEW_T), g2 = (long)tiles * ((n + 2 * FEW_T - 1) / (2 * FEW_T));
+    return g1 > 256 && (g2 <= 256 || g1 > 256 * per);
+}
+
 int launch_few_resid(hipStream_t st, const GemmArgs &a) {
     const int nc = (a.W.cols / QB + FEW_CB - 1) / FEW_CB, nck = (nc + FEW_NW - 1) / FEW_NW;
     if (!few_quantized(a.W) || a.units % 16 != 0 || a.out_stride % 4 != 0 || a.n <= 0 || nck > 4) return -1;
-    const dim3 g(a.units / 16, (a.n + FEW_T - 1) / FEW_T), b(64 * FEW_NW);
-#define FR(N)                                                                                   \
-    if (nck == N) {                                                                             \
-        if (a.W.dtype == DT_Q8) hipLaunchKernelGGL((k_few_resid<DT_Q8, N>), g, b, 0, st, a);    \
-        else hipLaunchKernelGGL((k_few_resid<DT_Q4, N>), g, b, 0, st, a);                       \
-        return 0;                                                                               \
+    const bool two = nck < 4 && few_two(a.units / 16, a.n, 1);
+    const dim3 g(a.units / 16, (a.n + FEW_T * (two ? 2 : 1) - 1) / (FEW_T * (two ? 2 : 1))), b(64 * FEW_NW);
+#define FR(N, TN)                                                                                   \
+    if (nck == N && two == (TN == 2)) {                                                             \
+        if (a.W.dtype == DT_Q8) hipLaunchKernelGGL((k_few_resid<DT_Q8, N, TN>), g, b, 0, st, a);    \
+        else hipLaunchKernelGGL((k_few_resid<DT_Q4, N, TN>), g, b, 0, st, a);                       \
+        return 0;                                                                                   \
     }
-    FR(1) FR(2) FR(3) FR(4)
+    FR(1, 1) FR(2, 1) FR(3, 1) FR(4, 1) FR(1, 2) FR(2, 2) FR(3, 2)
 #undef FR
     return -1;
 }
@@ -445,9 +493,13 @@ int launch_few_store(hipStream_t st, const GemmArgs &a, const NormIn &in) {
 int launch_few_swiglu(hipStream_t st, const GemmArgs &a, const NormIn &in) {
     if (!few_quantized(a.W) || a.W.cols > FEW_K || a.n <= 0 || a.units % SW_U != 0 || a.pair_off < a.units) return -1;
     if (!a.oq || !a.odx || !a.oxs) return -1;
-    const dim3 g(a.units / SW_U, (a.n + SW_T - 1) / SW_T), b(64 * FEW_NW);
-    if (a.W.dtype == DT_Q8) hipLaunchKernelGGL((k_few_swiglu<DT_Q8>), g, b, 0, st, a, in);
-    else hipLaunchKernelGGL((k_few_swiglu<DT_Q4>), g, b, 0, st, a, in);
+    const int tn = few_two(a.units / SW_U, a.n, 2) ? 2 : 1;
+    const dim3 g(a.units / SW_U, (a.n + SW_T * tn - 1) / (SW_T * tn)), b(64 * FEW_NW);
+#define FS(DT)                                                                                  \
+    if (tn == 2) hipLaunchKernelGGL((k_few_swiglu<DT, 2>), g, b, 0, st, a, in);                 \
+    else hipLaunchKernelGGL((k_few_swiglu<DT, 1>), g, b, 0, st, a, in);
+    if (a.W.dtype == DT_Q8) { FS(DT_Q8) } else { FS(DT_Q4) }
+#undef FS
     return 0;
 }
 

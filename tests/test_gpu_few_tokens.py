@@ -61,6 +61,13 @@ def test_products(shape, n):
     run(shape, n, False, 0)
 
 
+# two token tiles per workgroup in w1|w3 alone and in wo and w2, the last one
+# with a single token
+@pytest.mark.parametrize("shape,n", [("b", 81), ("d", 49), ("d", 97), ("b", 241)])
+def test_two_token_tiles(shape, n):
+    run(shape, n, True, 0)
+
+
 # a history inside the first tile, on a tile's edge, off it, of many key
 # ranges; rows that fill 64-row tiles to the last and past it, up to the four
 # the kernel takes and one more, which it does not
