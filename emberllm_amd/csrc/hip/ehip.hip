@@ -933,22 +933,24 @@ static int wait_step(EhipState *s, int ticket) {
     }
 }
 
+// A step without a graph is launched kernel by kernel, and the graph that the
+// next ones replay is captured and instantiated while it runs (0.2-0.45 ms of
+// host time, before the first kernel otherwise).
 static int run_step(EhipState *s) {
-    if (s->graph_mode) {
-        if (!s->gexec) {
-            HCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal), -1);
-            int rc = enq_step(s);
-            hipGraph_t g = nullptr;
-            hipError_t e = hipStreamEndCapture(s->st, &g);
-            if (rc) { if (g) (void)hipGraphDestroy(g); return -1; }
-            if (e != hipSuccess) { set_err("hipStreamEndCapture: %s", hipGetErrorString(e)); return -1; }
-            s->graph = g;
-            HCHK(hipGraphInstantiate(&s->gexec, g, nullptr, nullptr, 0), -1);
-        }
+    if (s->graph_mode && s->gexec) {
         HCHK(hipGraphLaunch(s->gexec, s->st), -1);
-    } else if (enq_step(s)) {
-        return -1;
+        return 0;
     }
+    if (enq_step(s)) return -1;
+    if (!s->graph_mode) return 0;
+    HCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal), -1);
+    int rc = enq_step(s);
+    hipGraph_t g = nullptr;
+    hipError_t e = hipStreamEndCapture(s->st, &g);
+    if (rc) { if (g) (void)hipGraphDestroy(g); return -1; }
+    if (e != hipSuccess) { set_err("hipStreamEndCapture: %s", hipGetErrorString(e)); return -1; }
+    s->graph = g;
+    HCHK(hipGraphInstantiate(&s->gexec, g, nullptr, nullptr, 0), -1);
     return 0;
 }
 
@@ -1385,13 +1387,13 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
     return 0;
 }
 
-// One prefill pass.  A shape's first pass is launched kernel by kernel and its
-// second captures the graph that it and later ones replay: each turn of a
-// conversation starts at another position, so most shapes run once, and
-// capturing and instantiating their launches (Qwen3-0.6B shape, 170 to 226
-// kernels) takes 0.4-0.6 ms of host time before the first kernel starts,
-// where the launches themselves hide behind the kernels.  Eager as well while
-// a layer's tensors are captured for inspection, or with graphs off.
+// One prefill pass.  A shape's first two passes are launched kernel by kernel,
+// and while the second runs the graph is captured that later ones replay.
+// Each turn of a conversation starts at another position, so most shapes run
+// once, and capturing and instantiating their launches (Qwen3-0.6B shape, 140
+// to 226 kernels) takes 0.4-0.6 ms of host time, where the launches themselves
+// hide behind the kernels.  Eager as well while a layer's tensors are captured
+// for inspection, or with graphs off.
 static int run_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass) {
     if (!s->graph_mode || s->pdbg_layer >= 0) return enq_prefill_pass(s, pos0, mt, last, pass);
     EhipState::PfGraph *hit = nullptr, *lru = &s->pfg[0];
@@ -1406,10 +1408,13 @@ static int run_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             s->pf_once[s->pf_once_next++ % PF_GRAPHS] = {pos0, mt, (int)last};
             return enq_prefill_pass(s, pos0, mt, last, pass);
         }
+        if (enq_prefill_pass(s, pos0, mt, last, pass)) return -1;
         hit = lru;
         graph_free(hit->sg);
         if (graph_capture(s, hit->sg, 1, [&]() { return enq_prefill_pass(s, pos0, mt, last, pass); })) return -1;
         hit->pos0 = pos0; hit->n = mt; hit->last = last;
+        hit->used = ++s->pf_clock;
+        return 0;
     }
     hit->used = ++s->pf_clock;
     HCHK(hipGraphLaunch(hit->sg.x, s->st), -1);
