@@ -338,7 +338,9 @@ __global__ __launch_bounds__(64 * FEW_NW) void k_few_qkv(GemmArgs a, NormIn in, 
 }
 
 // out = W . x (+ bias): 16-row tiles, eight waves over K, two of the rows per
-// wave to normalize.
+// wave to normalize.  16 tokens of the Qwen3-0.6B shape 6.8 us on 256
+// workgroups of 16 KB of weights (k_few_qkv 12.5 on 32), of which the
+// attention's QK-norm, RoPE and KV store take 3 back.
 constexpr int FEW_SW = 8;
 template <int DT>
 __global__ __launch_bounds__(64 * FEW_SW) void k_few_store(GemmArgs a, NormIn in) {
