@@ -111,7 +111,10 @@ __global__ __launch_bounds__(WG) void k_quant_rows(QuantRowsArgs a) {
 }
 
 // The rows behind an RMSNorm, in registers from the load to the store: thread
-// t holds elements 4 (t + 256 j) .. + 3, so eight lanes hold a block.  Bound
+// t holds elements 4 (t + 256 j) .. + 3, so eight lanes hold a block.  The
+// squares are summed in k_quant_rows's order (thread t elements t, t + 256,
+// ..., read a second time beside the first), so a row's bits do not depend on
+// which of the two kernels normalized it.  Bound
 // by its launch and memory round trip; k_quant_rows, which goes on with the
 // embedding, the SwiGLU and longer rows, stages them through LDS: Qwen3-0.6B
 // shape, 256 tokens 2468 -> 2428 us, 4000 tokens 14.97 -> 14.89 ms;
@@ -121,15 +124,19 @@ template <int N>
 __global__ __launch_bounds__(WG) void k_norm_rows(QuantRowsArgs a) {
     __shared__ float red[NWAVE];
     const int K = a.cols, nv = K / 4, nb = K / QB, b = blockIdx.x, tid = threadIdx.x;
+    const float *row = a.x + (size_t)b * a.x_stride;
+    float e[4 * N];
     f32x4 x[N], w[N];
 #pragma unroll
-    for (int j = 0; j < N; j++) x[j] = reinterpret_cast<const f32x4 *>(a.x + (size_t)b * a.x_stride)[min(tid + WG * j, nv - 1)];
+    for (int j = 0; j < 4 * N; j++) e[j] = row[min(tid + WG * j, K - 1)];
+#pragma unroll
+    for (int j = 0; j < N; j++) x[j] = reinterpret_cast<const f32x4 *>(row)[min(tid + WG * j, nv - 1)];
 #pragma unroll
     for (int j = 0; j < N; j++) w[j] = reinterpret_cast<const f32x4 *>(a.norm_w)[min(tid + WG * j, nv - 1)];
     float ss = 0.0f;
 #pragma unroll
-    for (int j = 0; j < N; j++)
-        if (tid + WG * j < nv) ss += (x[j].x * x[j].x + x[j].y * x[j].y) + (x[j].z * x[j].z + x[j].w * x[j].w);
+    for (int j = 0; j < 4 * N; j++)
+        if (tid + WG * j < K) ss += e[j] * e[j];
     const float scale = 1.0f / sqrtf(block_sum(ss, red) / (float)K + a.eps);   // model.c:50-55
 #pragma unroll
     for (int j = 0; j < N; j++) {
@@ -142,7 +149,7 @@ __global__ __launch_bounds__(WG) void k_norm_rows(QuantRowsArgs a) {
         const float id = d > 0.0f ? 1.0f / d : 0.0f;
         int c[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) c[e] = (int)fminf(fmaxf(roundf(v[e] * id), -127.0f), 127.0f);
+        for (int u = 0; u < 4; u++) c[u] = (int)fminf(fmaxf(roundf(v[u] * id), -127.0f), 127.0f);
         const int cs = sum8(c[0] + c[1] + c[2] + c[3]);
         if (i >= nv) continue;
         reinterpret_cast<uint32_t *>(a.qx + (size_t)b * K)[i] = ((uint32_t)c[0] & 0xffu) | (((uint32_t)c[1] & 0xffu) << 8) |
