@@ -26,6 +26,7 @@
 #include "kernels.h"
 #include "flimg.h"
 #include "gemm_epi.h"
+#include "f32_tile.h"
 
 namespace ehip {
 
@@ -242,15 +243,15 @@ __global__ __launch_bounds__(WG) void k_gemm_f32(GemmArgs a) {
     uint8_t *mine = lds + wave * WBYTES;
 
     // buffers over the tile's weight rows (EPI_SWIGLU: gate and up rows) and
-    // token rows: rows past the product's read as zeros, and a load's address is
-    // one lane offset plus a scalar
+    // token rows, each load inside them by its own offset (f32_load_offset: the
+    // row clamped to the buffer's last, the piece within the block) plus the
+    // block's scalar one (within a row); the buffers' range checks, which need
+    // not cover the scalar offset, decide nothing
     const float *w0 = reinterpret_cast<const float *>(a.W.q) + (size_t)u0 * K;
-    const int wbytes = min(OU, a.units - u0) * K * 4;
-    const auto bw = row_buffer(w0, wbytes);
-    const auto bu = row_buffer(w0 + (EPI == EPI_SWIGLU ? (size_t)a.pair_off * K : 0), wbytes);
-    const auto bx = row_buffer(a.xf + (size_t)t0 * K, min(RT, a.n - t0) * K * 4);
-    // rows lane / 8 + 8 i, i even and odd
-    const int lo0 = (lane >> 3) * K * 4 + 16 * ((lane & 7) ^ (lane >> 4)), lo1 = lo0 ^ 64;
+    const int wrows = min(OU, a.units - u0), xrows = min(RT, a.n - t0);
+    const auto bw = row_buffer(w0, wrows * K * 4);
+    const auto bu = row_buffer(w0 + (EPI == EPI_SWIGLU ? (size_t)a.pair_off * K : 0), wrows * K * 4);
+    const auto bx = row_buffer(a.xf + (size_t)t0 * K, xrows * K * 4);
     // pipeline: block b's fragments in fr[f], block b + 1 in st on its way to
     // LDS; past the last block the loads repeat it
     f32x4 st[LD], fr[2][4][MU + MT];
@@ -262,9 +263,9 @@ __global__ __launch_bounds__(WG) void k_gemm_f32(GemmArgs a) {
     auto load = [&](int i, int b) __attribute__((always_inline)) {
         const int k = min(b, b1 - 1) * QB * 4;
         constexpr int GU = EPI == EPI_SWIGLU ? 2 * MU : 4 * MU;   // 8-row groups of the first weight buffer
-        const auto v = i < GU ? __builtin_amdgcn_raw_buffer_load_b128(bw, i & 1 ? lo1 : lo0, 32 * i * K + k, 0)
-                     : i < 4 * MU ? __builtin_amdgcn_raw_buffer_load_b128(bu, i & 1 ? lo1 : lo0, 32 * (i - GU) * K + k, 0)
-                                  : __builtin_amdgcn_raw_buffer_load_b128(bx, i & 1 ? lo1 : lo0, 32 * (i - 4 * MU) * K + k, 0);
+        const auto v = i < GU ? __builtin_amdgcn_raw_buffer_load_b128(bw, f32_load_offset(lane, i, K, wrows), k, 0)
+                     : i < 4 * MU ? __builtin_amdgcn_raw_buffer_load_b128(bu, f32_load_offset(lane, i - GU, K, wrows), k, 0)
+                                  : __builtin_amdgcn_raw_buffer_load_b128(bx, f32_load_offset(lane, i - 4 * MU, K, xrows), k, 0);
         st[i] = __builtin_bit_cast(f32x4, v);
     };
     auto put = [&](int i) __attribute__((always_inline)) {

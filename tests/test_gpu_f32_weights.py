@@ -70,6 +70,21 @@ def test_prefill_products(shape, n):
     np.testing.assert_array_equal(got[1][0], xout)
 
 
+# a pass that fills its context, whose last tile ends behind the last row of
+# every buffer: the same logits as in a larger context
+@pytest.mark.parametrize("shape,n", [(SHAPES[0], 33), (SHAPES[1], 70), (SHAPES[2], 1001)], ids=lambda v: v[0] if isinstance(v, tuple) else str(v))
+def test_a_pass_that_fills_its_context(shape, n):
+    path = model(*shape)
+    ids = np.random.default_rng(n).integers(0, 320, n)
+    out = []
+    for ctx in (n, 1024):
+        eng = emberllm.Engine(path, ctx=ctx)
+        out.append(eng.prefill(ids))
+        eng.close()
+    assert np.isfinite(out[0]).all()
+    np.testing.assert_array_equal(out[0], out[1])
+
+
 # a row of 24 chunks (part of a wave), of 200, of 520 (two segments of 8 x 64
 # chunks, the second short, with the looped activation prologue) and the
 # widths of each segment size; the vocabulary's rows four to a wave
