@@ -395,6 +395,9 @@ static void graph_free(StepGraph &sg) {
 struct EhipState {
     EhipModel *m;
     int ctx, f16kv, esize, graph_mode;
+    // EHIP_GRAPH_TEST_FAIL=1 (a test hook): every graph's instantiation fails
+    // as if memory had run out
+    int graph_test_fail;
     hipStream_t st;
     void *kc, *vc;
     int *tokpos_d, *tokpos_h;   // {token, position, steps generated, API step ticket}
@@ -453,7 +456,7 @@ struct EhipState {
     float *att_ref;
     // device greedy loop: argmax partials, counter, generated tokens [ctx]
     float *am_val; int *am_idx; int *gen_tok;
-    hipGraph_t graph; hipGraphExec_t gexec;
+    StepGraph step;   // the API decode step
     // one hipGraph per prefill pass shape (first position, tokens, whether it
     // ends the prompt and so runs the head), least recently used evicted
     struct PfGraph { StepGraph sg; int pos0 = -1, n = 0, last = 0; unsigned long long used = 0; };
@@ -495,8 +498,20 @@ static int graph_capture(EhipState *s, StepGraph &sg, int steps, F enq) {
     if (rc) { if (g) (void)hipGraphDestroy(g); return -1; }
     if (e != hipSuccess) { set_err("hipStreamEndCapture: %s", hipGetErrorString(e)); return -1; }
     sg.g = g;
-    HCHK(hipGraphInstantiate(&sg.x, g, nullptr, nullptr, 0), -1);
+    const hipError_t ei = s->graph_test_fail ? hipErrorOutOfMemory : hipGraphInstantiate(&sg.x, g, nullptr, nullptr, 0);
+    if (ei != hipSuccess) { set_err("hipGraphInstantiate: %s", hipGetErrorString(ei)); return -1; }
     return 0;
+}
+
+// The graph of a step or pass that has just been launched kernel by kernel
+// and may still be running.  The launched work is good whatever becomes of
+// the graph, so where none can be had the state goes on without.
+template <class F>
+static void capture_behind(EhipState *s, StepGraph &sg, F enq) {
+    if (graph_capture(s, sg, 1, enq) == 0) return;
+    graph_free(sg);
+    (void)hipGetLastError();
+    s->graph_mode = 0;
 }
 
 static void *salloc(EhipState *s, size_t n, bool zero = false) {
@@ -510,8 +525,7 @@ static void *salloc(EhipState *s, size_t n, bool zero = false) {
 extern "C" void ehip_state_destroy(EhipState *s) {
     if (!s) return;
     (void)hipStreamSynchronize(s->st);
-    if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
-    if (s->graph) (void)hipGraphDestroy(s->graph);
+    graph_free(s->step);
     for (StepGraph &g : s->gen) graph_free(g);
     for (StepGraph &g : s->smp) graph_free(g);
     for (auto &pg : s->pfg) graph_free(pg.sg);
@@ -597,6 +611,7 @@ extern "C" EhipState *ehip_state_create(EhipModel *m, int ctx, int kv_fp16) {
     EhipState *s = new EhipState();  // value-initialised: every pointer starts null
     s->m = m; s->ctx = ctx; s->f16kv = kv_fp16 ? 1 : 0; s->esize = kv_fp16 ? 2 : 4;
     s->graph_mode = env_int("EHIP_GRAPH", 1);
+    s->graph_test_fail = env_int("EHIP_GRAPH_TEST_FAIL", 0);
     s->fw_spin = env_int("EHIP_FW_TEST_SPIN", ATT_DEC_FW_SPIN);
     s->tok_skew = env_int("EHIP_XMERGE_TEST_TOK", 0);
     if (hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking) != hipSuccess) {
@@ -937,20 +952,12 @@ static int wait_step(EhipState *s, int ticket) {
 // next ones replay is captured and instantiated while it runs (0.2-0.45 ms of
 // host time, before the first kernel otherwise).
 static int run_step(EhipState *s) {
-    if (s->graph_mode && s->gexec) {
-        HCHK(hipGraphLaunch(s->gexec, s->st), -1);
+    if (s->graph_mode && s->step.x) {
+        HCHK(hipGraphLaunch(s->step.x, s->st), -1);
         return 0;
     }
     if (enq_step(s)) return -1;
-    if (!s->graph_mode) return 0;
-    HCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal), -1);
-    int rc = enq_step(s);
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamEndCapture(s->st, &g);
-    if (rc) { if (g) (void)hipGraphDestroy(g); return -1; }
-    if (e != hipSuccess) { set_err("hipStreamEndCapture: %s", hipGetErrorString(e)); return -1; }
-    s->graph = g;
-    HCHK(hipGraphInstantiate(&s->gexec, g, nullptr, nullptr, 0), -1);
+    if (s->graph_mode) capture_behind(s, s->step, [&]() { return enq_step(s); });
     return 0;
 }
 
@@ -960,7 +967,10 @@ extern "C" float *ehip_forward(EhipState *s, int tok, int pos) {
     s->tokpos_h[2] = 0;
     for (int attempt = 0; attempt < 2; attempt++) {
         const int ticket = s->tokpos_h[3] = ++s->ticket;
-        if (run_step(s)) return nullptr;
+        if (run_step(s)) {
+            (void)hipStreamSynchronize(s->st);   // what was launched reads tokpos_h
+            return nullptr;
+        }
         if (wait_step(s, ticket)) return nullptr;
         int flag;
         memcpy(&flag, s->logits_h + s->m->cfg.vocab_size, 4);
@@ -1409,11 +1419,9 @@ static int run_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
             return enq_prefill_pass(s, pos0, mt, last, pass);
         }
         if (enq_prefill_pass(s, pos0, mt, last, pass)) return -1;
-        hit = lru;
-        graph_free(hit->sg);
-        if (graph_capture(s, hit->sg, 1, [&]() { return enq_prefill_pass(s, pos0, mt, last, pass); })) return -1;
-        hit->pos0 = pos0; hit->n = mt; hit->last = last;
-        hit->used = ++s->pf_clock;
+        capture_behind(s, lru->sg, [&]() { return enq_prefill_pass(s, pos0, mt, last, pass); });
+        lru->pos0 = pos0; lru->n = mt; lru->last = last;
+        lru->used = ++s->pf_clock;
         return 0;
     }
     hit->used = ++s->pf_clock;
@@ -1431,7 +1439,10 @@ extern "C" float *ehip_prefill(EhipState *s, const int *ids, int n, int start) {
         const int mt = std::min(s->pf_chunk, n - c0), pass = c0 / s->pf_chunk;
         const bool last = c0 + mt == n;
         HCHK(hipMemcpyAsync(s->ids_d, ids + c0, 4 * (size_t)mt, hipMemcpyHostToDevice, s->st), nullptr);
-        if (run_prefill_pass(s, start + c0, mt, last, pass)) return nullptr;
+        if (run_prefill_pass(s, start + c0, mt, last, pass)) {
+            (void)hipStreamSynchronize(s->st);   // what was launched reads ids and writes logits_h
+            return nullptr;
+        }
     }
     HCHK(hipStreamSynchronize(s->st), nullptr);
     return s->logits_h;
@@ -1473,10 +1484,7 @@ extern "C" int ehip_debug_buffer(EhipState *s, int which, void *host, uint64_t b
 
 static void drop_step_graphs(EhipState *s) {
     (void)hipStreamSynchronize(s->st);
-    if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
-    if (s->graph) (void)hipGraphDestroy(s->graph);
-    s->gexec = nullptr;
-    s->graph = nullptr;
+    graph_free(s->step);
     for (StepGraph &g : s->gen) graph_free(g);
     for (StepGraph &g : s->smp) graph_free(g);
 }
@@ -1563,8 +1571,9 @@ extern "C" int ehip_time_decode(EhipState *s, int pos0, int steps, float *ms) {
         const int pos = pos0 + i;
         s->tokpos_h[0] = (int)(((long)pos * 131 + 7) % V);
         s->tokpos_h[1] = pos;
-        if (run_step(s)) return -1;
+        const int rc = run_step(s);
         HCHK(hipStreamSynchronize(s->st), -1);
+        if (rc) return -1;
     }
     HCHK(hipEventRecord(s->ev1, s->st), -1);
     HCHK(hipEventSynchronize(s->ev1), -1);
