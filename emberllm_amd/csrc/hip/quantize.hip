@@ -3,8 +3,9 @@
 // quantize_tensor (src/quant.c:26-57) called by ember_quantize_file.
 //
 // fp32 rows stream from the caller's (mapped) host memory through pinned slots
-// of 1 MiB, one per host thread (QuantCall); the encoded blocks come back the
-// same way.  Each GPU thread encodes one 32-weight block with the reference's arithmetic
+// (QuantCall: one for a call of up to 24 MiB, one of 1 MiB per host thread for
+// longer ones); the encoded blocks come back the same way.  Each GPU thread
+// encodes one 32-weight block with the reference's arithmetic
 // (src/kernels.c:73-115), so the blocks equal the host quantizers' byte for
 // byte:
 //   Q8_0: amax over |x| (first maximum), d = amax/127, inverse from the
@@ -108,21 +109,31 @@ __global__ __launch_bounds__(256) void k_quant_blocks(const float *__restrict__ 
     }
 }
 
-// Up to PIECE_BLOCKS consecutive blocks of a job (its rows are contiguous in
-// both buffers, and a block never spans two).
-struct Piece { int job; size_t b0, n; };
-constexpr size_t PIECE_BLOCKS = 8192;                  // 1 MiB of fp32
+// A piece: blocks of the jobs of one encoding, in the jobs' order (a job's rows
+// are contiguous in both buffers, and a block never spans two), so one launch
+// and one DMA each way serve many small matrices: 100 of 32 x 64 2.5 ms with a
+// piece each, 0.2 together.
+struct Segment { int job; size_t b0, n; };
+struct Piece { size_t seg, nseg, blocks; int dtype; };
 constexpr int64_t ROW_MAX = (int64_t)32 << 20;         // bytes of a row at most
 constexpr int QUANT_STREAMS = 4;
+// Calls of up to ALONE_BLOCKS (24 MiB of fp32) are a piece per encoding, which
+// the calling thread copies itself; longer ones go in pieces of
+// PIECE_BLOCKS (1 MiB) over several threads, whose start, streams and smaller
+// copies cost about 1 ms a call.  One matrix, one piece against pieces over
+// threads: 4 MiB 0.4 ms against 1.6, 12 MiB 0.75 against 1.5, 24 MiB 1.4
+// against 1.9, 32 MiB 2.2 against 2.2; from 40 MiB on one piece falls to 20 ms.
+constexpr size_t ALONE_BLOCKS = 196608, PIECE_BLOCKS = 8192;
 
 // The call's pieces and staging: each worker thread has a pinned and a device
 // slot of one piece each way, and takes the next piece when its last is done:
 // copy in, DMA, one launch, DMA back, copy out.  The workers' host copies, the
-// DMAs and the kernels overlap, and nothing is sized by the matrices: pinning
-// dominates a call on a few of them (the feed-forward matrices of a 0.6B
-// layer, 37.7 MB: three pinned slots of 32 MB 6.9 ms a call).
+// DMAs and the kernels overlap, and a long call's slots are not sized by its
+// matrices: pinning dominates a call on a few of them (the feed-forward
+// matrices of a 0.6B layer, 37.7 MB: three pinned slots of 32 MB 6.9 ms a call).
 struct QuantCall {
     const EhipQuantJob *jobs;
+    std::vector<Segment> segs;
     std::vector<Piece> pieces;
     size_t in_bytes = 0, out_bytes = 0;   // of a slot
     int workers = 0;
@@ -130,21 +141,31 @@ struct QuantCall {
     hipStream_t st[QUANT_STREAMS] = {};
     std::vector<hipEvent_t> ev;
     std::atomic<size_t> next{0};
-    std::atomic<bool> failed{false};
+    std::atomic<const char *> failure{nullptr};
 
-    bool open(const EhipQuantJob *j, int n_jobs) {
+    bool open(const EhipQuantJob *j, int n_jobs, size_t total) {
         jobs = j;
+        const bool alone = total <= ALONE_BLOCKS;
+        const size_t piece = alone ? ALONE_BLOCKS : PIECE_BLOCKS;
         size_t most = 0;
-        for (int i = 0; i < n_jobs; i++) {
-            const size_t nblk = (size_t)jobs[i].rows * (jobs[i].cols / 32);
-            for (size_t b = 0; b < nblk; b += PIECE_BLOCKS) {
-                pieces.push_back({ i, b, std::min(PIECE_BLOCKS, nblk - b) });
-                most = std::max(most, pieces.back().n);
+        for (int dtype : { DT_Q8, DT_Q4 })
+            for (int i = 0; i < n_jobs; i++) {
+                const size_t nblk = jobs[i].dtype == dtype ? (size_t)jobs[i].rows * (jobs[i].cols / 32) : 0;
+                for (size_t b = 0; b < nblk;) {
+                    if (pieces.empty() || pieces.back().blocks == piece || pieces.back().dtype != dtype)
+                        pieces.push_back({ segs.size(), 0, 0, dtype });
+                    Piece &p = pieces.back();
+                    const size_t n = std::min(piece - p.blocks, nblk - b);
+                    segs.push_back({ i, b, n });
+                    p.nseg++;
+                    p.blocks += n;
+                    b += n;
+                    most = std::max(most, p.blocks);
+                }
             }
-        }
         in_bytes = most * 128;
         out_bytes = (most * 34 + 127) & ~(size_t)127;
-        workers = (int)std::min<size_t>(staging_threads(), pieces.size());
+        workers = alone ? 1 : (int)std::min<size_t>(staging_threads(), pieces.size());
         const size_t bytes = (in_bytes + out_bytes) * workers;
         if (hipHostMalloc(reinterpret_cast<void **>(&pin), bytes, hipHostMallocDefault) != hipSuccess) { pin = nullptr; return false; }
         if (hipMalloc(reinterpret_cast<void **>(&dev), bytes) != hipSuccess) { dev = nullptr; return false; }
@@ -167,28 +188,37 @@ struct QuantCall {
             if (s) (void)hipStreamDestroy(s);
     }
 
-    bool piece(int w, const Piece &p) {
-        const EhipQuantJob &j = jobs[p.job];
-        const size_t ob = j.dtype == DT_Q8 ? 34 : 18, slot = (in_bytes + out_bytes) * w;
+    // piece p through worker w's slot; what failed, or null
+    const char *piece(int w, const Piece &p) {
+        const size_t ob = p.dtype == DT_Q8 ? 34 : 18, slot = (in_bytes + out_bytes) * w;
         uint8_t *pin_in = pin + slot, *pin_out = pin_in + in_bytes, *dev_in = dev + slot, *dev_out = dev_in + in_bytes;
         const hipStream_t s = st[w % QUANT_STREAMS];
-        memcpy(pin_in, reinterpret_cast<const uint8_t *>(j.src) + p.b0 * 128, p.n * 128);
-        if (hipMemcpyAsync(dev_in, pin_in, p.n * 128, hipMemcpyHostToDevice, s) != hipSuccess) return false;
-        const int grid = (int)((p.n + 255) / 256);
+        const Segment *g0 = &segs[p.seg], *g1 = g0 + p.nseg;
+        uint8_t *in = pin_in;
+        for (const Segment *g = g0; g < g1; in += g->n * 128, g++)
+            memcpy(in, reinterpret_cast<const uint8_t *>(jobs[g->job].src) + g->b0 * 128, g->n * 128);
+        bool ok = hipMemcpyAsync(dev_in, pin_in, p.blocks * 128, hipMemcpyHostToDevice, s) == hipSuccess;
+        const int grid = (int)((p.blocks + 255) / 256);
         const float *x = reinterpret_cast<const float *>(dev_in);
         uint16_t *o = reinterpret_cast<uint16_t *>(dev_out);
-        if (j.dtype == DT_Q8) k_quant_blocks<DT_Q8><<<grid, 256, 0, s>>>(x, p.n, o);
-        else k_quant_blocks<DT_Q4><<<grid, 256, 0, s>>>(x, p.n, o);
-        if (hipGetLastError() != hipSuccess || hipMemcpyAsync(pin_out, dev_out, p.n * ob, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipEventRecord(ev[w], s) != hipSuccess || hipEventSynchronize(ev[w]) != hipSuccess)
-            return false;
-        memcpy(static_cast<uint8_t *>(j.dst) + p.b0 * ob, pin_out, p.n * ob);
-        return true;
+        if (p.dtype == DT_Q8) k_quant_blocks<DT_Q8><<<grid, 256, 0, s>>>(x, p.blocks, o);
+        else k_quant_blocks<DT_Q4><<<grid, 256, 0, s>>>(x, p.blocks, o);
+        ok = hipGetLastError() == hipSuccess && ok;
+        ok = ok && hipMemcpyAsync(pin_out, dev_out, p.blocks * ob, hipMemcpyDeviceToHost, s) == hipSuccess &&
+             hipEventRecord(ev[w], s) == hipSuccess;
+        if (!ok) return "requantizer: queueing a slot's copies or kernels failed";
+        if (hipEventSynchronize(ev[w]) != hipSuccess) return "requantizer: waiting for a slot failed";
+        const uint8_t *out = pin_out;
+        for (const Segment *g = g0; g < g1; out += g->n * ob, g++)
+            memcpy(static_cast<uint8_t *>(jobs[g->job].dst) + g->b0 * ob, out, g->n * ob);
+        return nullptr;
     }
+    // what fails first ends every worker at its next piece; the destructor
+    // waits for what is on its way
     void work(int w) {
-        if (hipSetDevice(0) != hipSuccess) failed = true;
-        for (size_t i; !failed && (i = next.fetch_add(1)) < pieces.size();)
-            if (!piece(w, pieces[i])) failed = true;
+        if (hipSetDevice(0) != hipSuccess) failure = "hipSetDevice(0) failed: no usable GPU";
+        for (size_t i; !failure && (i = next.fetch_add(1)) < pieces.size();)
+            if (const char *e = piece(w, pieces[i])) failure = e;
     }
     bool run() {
         std::vector<std::thread> ts;
@@ -198,7 +228,7 @@ struct QuantCall {
         }
         work(0);
         for (std::thread &t : ts) t.join();
-        return !failed;
+        return !failure;
     }
 };
 
@@ -228,9 +258,9 @@ extern "C" int ehip_quantize_rows(const EhipQuantJob *jobs, int n_jobs) {
     if (hipSetDevice(0) != hipSuccess) { set_error_text("hipSetDevice(0) failed: no usable GPU"); return -1; }
     try {
         QuantCall q;
-        if (!q.open(jobs, n_jobs)) { set_error_text("requantizer: allocating the staging buffers failed"); return -1; }
+        if (!q.open(jobs, n_jobs, total / 128)) { set_error_text("requantizer: allocating the staging buffers failed"); return -1; }
         if (q.run()) return 0;
-        set_error_text("requantizer: a piece's copies or kernel failed");
+        set_error_text(q.failure.load());
     } catch (const std::exception &) {
         set_error_text("requantizer: out of host memory");
     }

@@ -93,6 +93,31 @@ def test_quantize_rows_many_jobs_and_slot_cycles():
         assert np.array_equal(g[idx], want), (x.shape, dt)
 
 
+@pytest.mark.parametrize("alone", [True, False])
+def test_quantize_rows_small_jobs_share_pieces(alone):
+    """Many small jobs of both encodings, which travel together, jobs without
+    rows among them, in a call that is one piece per encoding and in one of
+    many pieces, whose borders fall inside the jobs: the blocks of every job,
+    and no byte beside them."""
+    rng = np.random.default_rng(31)
+    q8, q4 = _native.DT_Q8_0, _native.DT_Q4_0
+    big = [] if alone else [(7000, 1024, q8)]
+    shapes = [(int(rng.integers(1, 9)), 32 * int(rng.integers(1, 6)), q8) for _ in range(300)] + \
+             [(0, 64, q8), (1030, 256, q8), (5, 32, q8), (0, 32, q4)] + big + \
+             [(int(rng.integers(1, 9)), 32 * int(rng.integers(1, 6)), rng.choice([q8, q4])) for _ in range(300)]
+    mats = [(rng.standard_normal((r, c)).astype(np.float32), int(dt)) for r, c, dt in shapes]
+    outs = [np.full(x.shape[0] * x.shape[1] // 32 * BS[dt] + 64, 0xA5, np.uint8) for x, dt in mats]
+    jobs = (_native.EhipQuantJob * len(mats))()
+    for j, ((x, dt), o) in enumerate(zip(mats, outs)):
+        jobs[j] = _native.EhipQuantJob(x.ctypes.data, x.shape[0], x.shape[1], dt, o.ctypes.data + 32)
+    assert lib().ehip_quantize_rows(jobs, len(mats)) == 0, _native.last_error()
+    for (x, dt), o in zip(mats, outs):
+        assert (o[:32] == 0xA5).all() and (o[-32:] == 0xA5).all(), (x.shape, dt)
+        got = o[32:-32].reshape(x.shape[0], x.shape[1] // 32 * BS[dt])
+        rows = np.arange(x.shape[0]) if x.shape[0] < 2000 else rng.integers(0, x.shape[0], 300)   # (the host's is slow here)
+        np.testing.assert_array_equal(got[rows], host_blocks(x[rows], dt))
+
+
 def test_quantize_rows_rejects_bad_jobs():
     x = np.zeros((2, 48), np.float32)
     o = np.zeros(200, np.uint8)
