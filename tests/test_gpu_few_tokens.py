@@ -23,14 +23,19 @@ def model(name, dim, hidden, heads, kv, hd, dtype, **kw):
     return configs.model_path("few_" + name, cfg)
 
 
-# K of 3, 18, 28 and 32 blocks in the normalized products, of 4 to 160 in wo
-# and w2; 1, 3, 7 and 2 query heads per kv head
+# K of 3, 8, 9, 18, 28 and 32 blocks in the normalized products, of 4 to 257
+# in wo and w2; 1, 2, 3 and 7 query heads per kv head
 SHAPES = {
     "a": ("a", 96, 1056, 2, 2, 64, Q8, dict(rope=_native.ROPE_INTERLEAVED)),
     "b": ("b", 576, 1536, 9, 3, 64, Q4, dict(bias=1)),
     "c": ("c", 896, 5120, 14, 2, 64, Q8, dict(bias=1, norm=1)),
     "d": ("d", 1024, 3072, 16, 8, 128, Q8, dict(norm=1)),
     "e": ("e", 1024, 1024, 4, 2, 128, Q4, dict(norm=1)),
+    # raw rows with a bias and interleaved RoPE; w2 of the most inputs, four
+    # chunks per wave, and of one block more, which the staged kernels take
+    "f": ("f", 256, 8192, 4, 2, 128, Q8, dict(bias=1, rope=_native.ROPE_INTERLEAVED)),
+    "g": ("g", 288, 8192, 3, 1, 128, Q4, dict(bias=1, norm=1, rope=_native.ROPE_INTERLEAVED)),
+    "h": ("h", 256, 8224, 4, 2, 64, Q8, dict()),
 }
 
 
@@ -74,6 +79,7 @@ def test_two_token_tiles(shape, n):
 @pytest.mark.parametrize("shape,n,start,kv16", [("a", 1, 1, False), ("a", 64, 640, True), ("b", 22, 129, False), ("b", 85, 1500, True),
                                                 ("c", 36, 63, True), ("c", 37, 640, False), ("d", 23, 517, True), ("d", 128, 1900, False),
                                                 ("d", 2, 126, False), ("d", 16, 250, True), ("d", 1, 63, False), ("d", 9, 64, True),
-                                                ("e", 33, 65, True), ("e", 9, 2000, False)])
+                                                ("e", 33, 65, True), ("e", 9, 2000, False), ("f", 16, 250, True),
+                                                ("g", 7, 63, False)])
 def test_attention_behind_a_history(shape, n, start, kv16):
     run(shape, n, kv16, start)
