@@ -362,7 +362,8 @@ constexpr size_t PF_SCORES_MAX = (size_t)1 << 30;   // bytes of attention scores
 // inputs keeps one sequential block sum per output in the prefill GEMMs, so
 // with exact-order attention its prefill matches the reference's
 // deterministic build to rounding: its passes of up to PF_EXACT_KEYS keys
-// use the exact-order kernels.  Wider models split their longer block sums
+// use the exact-order kernels (F32 weights add in k_gemm_f32's order; none of
+// their inputs is quantized, so that difference is rounding too).  Wider models split their longer block sums
 // over pipelines (and sum decode products across lanes), so they run at the
 // reference builds' own noise floor in any case: their attention runs on
 // the matrix cores at every length (the one-kernel exact form, once the
@@ -1402,7 +1403,9 @@ static int enq_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass)
 // Each turn of a conversation starts at another position, so most shapes run
 // once, and capturing and instantiating their launches (Qwen3-0.6B shape, 140
 // to 226 kernels) takes 0.4-0.6 ms of host time, where the launches themselves
-// hide behind the kernels.  Eager as well while a layer's tensors are captured
+// hide behind the kernels.  A second pass shorter than its capture waits for it
+// (stories110M, 2 tokens: 327 us, then 357-444, then 334; SmolLM2-135M 741,
+// 734-982, 742; from 16 tokens of Qwen3-0.6B on it hides).  Eager as well while a layer's tensors are captured
 // for inspection, or with graphs off.
 static int run_prefill_pass(EhipState *s, int pos0, int mt, bool last, int pass) {
     if (!s->graph_mode || s->pdbg_layer >= 0) return enq_prefill_pass(s, pos0, mt, last, pass);

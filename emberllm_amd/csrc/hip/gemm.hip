@@ -115,12 +115,12 @@ __global__ __launch_bounds__(WG) void k_quant_rows(QuantRowsArgs a) {
 // t holds elements 4 (t + 256 j) .. + 3, so eight lanes hold a block.  The
 // squares are summed in k_quant_rows's order (thread t elements t, t + 256,
 // ..., read a second time beside the first), so a row's bits do not depend on
-// which of the two kernels normalized it.  Bound
-// by its launch and memory round trip; k_quant_rows, which goes on with the
-// embedding, the SwiGLU and longer rows, stages them through LDS: Qwen3-0.6B
-// shape, 256 tokens 2468 -> 2428 us, 4000 tokens 14.97 -> 14.89 ms;
-// SmolLM2-135M 512 tokens 1971 -> 1893, Qwen2.5-0.5B (8 layers) 257 tokens 640
-// -> 624, stories110M F32 200 tokens 882 -> 838.
+// which of the two kernels normalized it.  Bound by its launch and memory
+// round trip; k_quant_rows, which goes on with the embedding, the SwiGLU and
+// longer rows, stages them through LDS: Qwen3-0.6B shape, 256 tokens 2468 ->
+// 2428 us, 4000 tokens 14.97 -> 14.89 ms; SmolLM2-135M 512 tokens 1971 -> 1893,
+// Qwen2.5-0.5B (8 layers) 257 tokens 640 -> 624, stories110M F32 200 tokens 882
+// -> 838.
 template <int N>
 __global__ __launch_bounds__(WG) void k_norm_rows(QuantRowsArgs a) {
     __shared__ float red[NWAVE];
